@@ -27,7 +27,7 @@ OUT = PKG / "libgrimoire_moe.so"
 OBJ = PKG / "_build"
 
 SOURCES = ["router.hip", "gemv.hip", "gemv_f0.hip", "gemv_f3.hip", "gemv_f4.hip", "gemv_f6.hip",
-           "gemv_f64.hip", "dispatch.hip", "gemm.hip", "gemm_i8.hip", "ingest.hip",
+           "gemv_f64.hip", "dispatch.hip", "gemm.hip", "gemm_i8.hip", "gemm_wreg.hip", "ingest.hip",
            "tiered.hip", "elementwise.hip", "gemv_grouped.hip", "gemv_mx.hip", "api.cpp", "forward.cpp", "heat.cpp"]
 # host-only sources (x86 intrinsics, threads): the C++ compiler, not hipcc
 HOST_SOURCES = ["cpu_experts.cc"]

@@ -121,6 +121,43 @@ __global__ __launch_bounds__(1024) void disp_scan(int E, int32_t* __restrict__ c
     if (threadIdx.x == 0 && n_tiles_out) *n_tiles_out = carry[1];
 }
 
+// disp_scan with descriptor lists in place of the tile table (one thread
+// per expert).
+__global__ __launch_bounds__(kTileListMaxE) void disp_scan_lists(int E, const int32_t* __restrict__ counts,
+                                                                 int32_t* __restrict__ offsets, TileLists l) {
+    __shared__ int32_t wsum[kTileListMaxE / 64][3];
+    const int e = threadIdx.x, lane = e & 63, wv = e >> 6;
+    const int c = e < E ? counts[e] : 0;
+    const int nt[2] = {(c + l.mc[0] - 1) / l.mc[0], (c + l.mc[1] - 1) / l.mc[1]};
+    int v[3] = {c, nt[0], nt[1]};
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int a = __shfl_up(v[q], off, 64);
+            if (lane >= off) v[q] += a;
+        }
+    if (lane == 63)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) wsum[wv][q] = v[q];
+    __syncthreads();
+    int tot[3] = {0, 0, 0};
+    for (int w = 0; w < kTileListMaxE / 64; ++w)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            v[q] += w < wv ? wsum[w][q] : 0;
+            tot[q] += wsum[w][q];
+        }
+    const int r0 = v[0] - c;
+    if (e < E) offsets[e] = r0;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        for (int i = 0; i < nt[q]; ++i)
+            l.d[q][v[q + 1] - nt[q] + i] = TileDesc{e, r0 + i * l.mc[q], min(l.mc[q], c - i * l.mc[q]), i};
+        if (e == 0) l.n[q] = tot[q + 1];
+    }
+}
+
 __global__ __launch_bounds__(kDispThreads) void disp_rank(const int32_t* __restrict__ ids, int R,
                                                           int E, int K,
                                                           const int32_t* __restrict__ bbase,
@@ -279,7 +316,11 @@ hipError_t dispatch_launch(hipStream_t st, const DispatchArgs& a) {
     // T > 0 here (the callers return before), so nb >= 1
     hipLaunchKernelGGL(disp_colscan, dim3((a.E + kColExperts - 1) / kColExperts),
                        dim3(kColExperts * kColSlices), 0, st, bcount, nb, a.E, a.counts);
-    if (!a.tile_e && a.E <= kRankScanMaxE && nb > 0) {
+    if (a.lists.n) {
+        hipLaunchKernelGGL(disp_scan_lists, dim3(1), dim3(kTileListMaxE), 0, st, a.E, a.counts, a.offsets, a.lists);
+        hipLaunchKernelGGL(disp_rank, dim3(nb), dim3(kDispThreads), 0, st, a.ids, R, a.E, a.K, bcount, a.offsets,
+                           a.inverse, a.perm_token);
+    } else if (!a.tile_e && a.E <= kRankScanMaxE && nb > 0) {
         // no tile table: the rank blocks form the offsets themselves
         hipLaunchKernelGGL(disp_rank_scan, dim3(nb), dim3(kDispThreads), 0, st, a.ids, R, a.E, a.K, bcount,
                            a.counts, a.offsets, a.inverse, a.perm_token, a.mc, ntiles);

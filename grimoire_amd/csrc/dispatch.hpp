@@ -5,6 +5,20 @@
 
 namespace grim {
 
+// Row tiles of the routed rows as descriptors: one 16-byte load tells a
+// work-group its expert, first row, row count and the tile's index inside
+// the expert.  Two lists (tiles of at most mc[0] and of mc[1] rows) for
+// products that tile the same rows differently.
+struct TileDesc {
+    int32_t e, r0, rows, mb;
+};
+struct TileLists {
+    TileDesc* d[2];
+    int mc[2];
+    int32_t* n;             // [2] live descriptors of each list
+};
+constexpr int kTileListMaxE = 1024;
+
 struct DispatchArgs {
     const int32_t* ids;     // [T*K]
     int T, K, E, H;
@@ -20,6 +34,7 @@ struct DispatchArgs {
     int32_t* tile_mb;
     int tmax, mc;
     void* workspace;        // dispatch_workspace_bytes
+    TileLists lists = {};   // E <= kTileListMaxE; in place of tile_e / tile_mb
 };
 
 struct CombineArgs {

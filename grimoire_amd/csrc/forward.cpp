@@ -22,6 +22,7 @@
 #include "dispatch.hpp"
 #include "gemm.hpp"
 #include "gemm_i8.hpp"
+#include "gemm_wreg.hpp"
 #include "gemv_grouped.hpp"
 #include "gemv_mx.hpp"
 #include "gemv.hpp"
@@ -108,7 +109,17 @@ struct Plan {
     int gv_tmax;
     float *gv_h, *gv_hsh;
     uint32_t *gv_xf, *gv_hf, *gv_hfsh;   // formatted activation rows
+    // register-weight products (gemm_wreg.hip): row tiles, route ->
+    // token map, bf16 activation planes
+    TileDesc* wr_tiles[2];    // gate_up's, down's
+    int wr_tmax[2];
+    int32_t *wr_live, *wr_perm, *wr_lo;
+    uint16_t *wr_x, *wr_h, *wr_hsh;
 };
+
+// What a call's workspace holds: the slot kernels, the grouped GEMM / GEMV
+// or the register-weight products.
+enum class PlanKind { kSlots, kGrouped, kWreg };
 
 // MXFP4 rows of the matrix-core grouped GEMV's length (gvm_padded_k):
 // payload K'/2, K'/32 scale bytes per row, K' = gvm_padded_k(K) >= K.
@@ -148,7 +159,35 @@ bool gv_ok(const grim_moe_layer* L) {
            (!pad || gvm_shape_ok(H, I));
 }
 
-size_t carve(const grim_moe_layer* L, int T, bool gemv, char* base, Plan& p) {
+// The register-weight products cover this layer at T tokens.
+bool wreg_ok(const grim_moe_layer* L, int T) {
+    const int f = L->gate_up.fmt, H = L->cfg.hidden, I = L->cfg.inter;
+    auto ok = [&](const grim_quant_weight& w, int rows, int K) { return w.fmt == f && wreg_weight_ok(w, rows, K); };
+    // (the token rows are gathered through 32-bit offsets)
+    return ok(L->gate_up, 2 * I, H) && ok(L->down, H, I) &&
+           (!L->has_shared || (ok(L->shared_gate_up, 2 * I, H) && ok(L->shared_down, H, I))) &&
+           L->cfg.num_experts <= kTileListMaxE && int64_t(T) * wreg_x_planes(f) * wreg_kpad(f, H) * 2 < 0x7FFFFFFF;
+}
+
+// ... and the call takes them: MXFP4 and bf16 experts wherever the grouped
+// GEMM would run (1000 tokens of 128 MXFP4 experts, H = I = 2880: 1300 ->
+// 660 us a layer; 150 tokens of 64 bf16 experts: 299 -> 231 us); INT4 experts
+// above 64 routes (fewer stay with the slot kernels) up to the two routes per
+// expert that INT4 batches are taken for, where the vector-ALU grouped GEMV
+// ran (20 tokens x top-8 of 128, H 2048, I 768: 304 -> 87 us).
+bool use_wreg(const grim_moe_layer* L, int T, int regime) {
+    const int64_t R = int64_t(T) * L->cfg.top_k;
+    const int f = L->gate_up.fmt;
+    if (!wreg_ok(L, T)) return false;
+    if (f == GRIM_FMT_INT4 || f == GRIM_FMT_INT4_F16)
+        return regime == 0 && R > 64 && R <= 2 * int64_t(L->cfg.num_experts);
+    if (regime == 2) return true;
+    return regime == 0 && !use_gemv(L, T, 0) &&
+           !(f == GRIM_FMT_MXFP4 && R <= 2 * int64_t(L->cfg.num_experts) && gv_ok(L));
+}
+
+size_t carve(const grim_moe_layer* L, int T, PlanKind kind, char* base, Plan& p) {
+    const bool gemv = kind == PlanKind::kSlots;
     const auto& c = L->cfg;
     const int E = c.num_experts, K = c.top_k, H = c.hidden, I = c.inter;
     const int64_t R = int64_t(T) * K;
@@ -168,6 +207,28 @@ size_t carve(const grim_moe_layer* L, int T, bool gemv, char* base, Plan& p) {
         p.hf = cv.take<uint32_t>(size_t(T) * fmt_words((K + (sh ? 1 : 0)) * I));
         p.xf = cv.take<uint32_t>(size_t(T) * xf_words(H));
         p.hrep = T == 1 ? cv.take<float>(size_t(kSyncCopies) * fused_h_stride(K, I)) : nullptr;
+    } else if (kind == PlanKind::kWreg) {
+        const int f = L->gate_up.fmt;
+        const int64_t hp = wreg_kpad(f, H), ip = wreg_kpad(f, I);
+        p.disp_ws = cv.take<char>(dispatch_workspace_bytes(T, K, E));
+        p.logits2 = cv.take<float>(size_t(T) * E);
+        const size_t wib = router_wimg_bytes(T, E, H);
+        p.wimg = wib ? static_cast<void*>(cv.take<char>(wib)) : nullptr;
+        p.counts = cv.take<int32_t>(E);
+        p.offsets = cv.take<int32_t>(E);
+        p.inverse = cv.take<int32_t>(R);
+        for (int q = 0; q < 2; ++q) {
+            p.wr_tmax[q] = int(std::min<int64_t>(R, E + R / wreg_mc(f, q == 0)));
+            p.wr_tiles[q] = cv.take<TileDesc>(p.wr_tmax[q]);
+        }
+        p.wr_live = cv.take<int32_t>(2);
+        p.wr_perm = cv.take<int32_t>(R);
+        p.wr_lo = cv.take<int32_t>(T);
+        p.wr_x = cv.take<uint16_t>(size_t(T) * wreg_x_planes(f) * hp);
+        p.wr_h = cv.take<uint16_t>(R * 2 * ip);
+        p.wr_hsh = sh ? cv.take<uint16_t>(size_t(T) * 2 * ip) : nullptr;
+        p.yperm = cv.take<float>(R * H);
+        p.ysh = sh ? cv.take<float>(size_t(T) * H) : nullptr;
     } else {
         const size_t dws = dispatch_workspace_bytes(T, K, E);
         p.disp_ws = cv.take<char>(dws);
@@ -224,9 +285,10 @@ size_t carve(const grim_moe_layer* L, int T, bool gemv, char* base, Plan& p) {
 extern "C" size_t grimoire_moe_forward_workspace_bytes(const grim_moe_layer* L, int tokens) {
     if (!L || tokens <= 0) return 0;
     Plan p{};
-    const size_t a = carve(L, tokens, true, nullptr, p);
-    const size_t b = carve(L, tokens, false, nullptr, p);
-    return a > b ? a : b;
+    const size_t a = carve(L, tokens, PlanKind::kSlots, nullptr, p);
+    const size_t b = carve(L, tokens, PlanKind::kGrouped, nullptr, p);
+    const size_t c = wreg_ok(L, tokens) ? carve(L, tokens, PlanKind::kWreg, nullptr, p) : 0;
+    return std::max(std::max(a, b), c);
 }
 
 extern "C" int grimoire_moe_router_logits(void*, const float*, const float*, float*, int, int, int);
@@ -459,10 +521,84 @@ static int forward_gv(hipStream_t st, const grim_moe_layer* L, const Plan& p, co
     return GRIM_OK;
 }
 
+// Register-weight products (a few to a few hundred rows per expert): routes
+// -> counts, offsets, tile table and token map -> x as bf16 planes ->
+// gate_up + SwiGLU (h as a bf16 pair per route) -> down (fp32 rows per
+// route) -> combine.
+static int forward_wreg(hipStream_t st, const grim_moe_layer* L, const Plan& p, const float* x, float* y,
+                        int tokens, const uint16_t* shared_gate_w) {
+    const auto& c = L->cfg;
+    const int E = c.num_experts, K = c.top_k, H = c.hidden, I = c.inter, f = L->gate_up.fmt;
+    const bool sh = L->has_shared;
+    DispatchArgs da{};
+    da.ids = p.rex;
+    da.T = tokens;
+    da.K = K;
+    da.E = E;
+    da.counts = p.counts;
+    da.offsets = p.offsets;
+    da.inverse = p.inverse;
+    da.perm_token = p.wr_perm;
+    da.workspace = p.disp_ws;
+    da.lists = TileLists{{p.wr_tiles[0], p.wr_tiles[1]}, {wreg_mc(f, true), wreg_mc(f, false)}, p.wr_live};
+    hipError_t e = dispatch_launch(st, da);
+    if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
+    e = wreg_format_launch(st, f, x, tokens, H, p.wr_x, p.wr_lo);
+    if (e == hipSuccess && sh && shared_gate_w) e = rowdot_sigmoid_launch(st, x, shared_gate_w, p.gate, tokens, H);
+    if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
+    WregArgs g{};
+    g.w = make_view(L->gate_up);
+    g.w_sh = sh ? make_view(L->shared_gate_up) : g.w;
+    g.N = I;
+    g.K = H;
+    g.A = g.A_sh = p.wr_x;
+    g.a_rows = g.a_rows_sh = tokens;
+    g.a_lo = p.wr_lo;
+    g.map = p.wr_perm;
+    g.h = p.wr_h;
+    g.h_sh = p.wr_hsh;
+    g.tiles = p.wr_tiles[0];
+    g.n_live = p.wr_live;
+    g.max_tiles = p.wr_tmax[0];
+    g.T_sh = sh ? tokens : 0;
+    e = wreg_launch(st, f, g, true);
+    if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
+    WregArgs d = g;
+    d.w = make_view(L->down);
+    d.w_sh = sh ? make_view(L->shared_down) : d.w;
+    d.N = H;
+    d.K = I;
+    d.A = p.wr_h;
+    d.A_sh = p.wr_hsh;
+    d.a_rows = int64_t(tokens) * K;
+    d.map = nullptr;
+    d.tiles = p.wr_tiles[1];
+    d.n_live = p.wr_live + 1;
+    d.max_tiles = p.wr_tmax[1];
+    d.y = p.yperm;
+    d.y_sh = p.ysh;
+    e = wreg_launch(st, f, d, false);
+    if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
+    CombineArgs cb{p.yperm, 0, p.inverse, p.rwt, p.ysh, 0, (sh && shared_gate_w) ? p.gate : nullptr,
+                   y, tokens, K, H};
+    e = combine_launch(st, cb);
+    if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
+    return GRIM_OK;
+}
+
 static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_params* rp,
                         const uint16_t* shared_gate_w, const float* x, float* y, int tokens,
                         int32_t* out_expert, float* out_weight, int regime, void* workspace,
                         size_t workspace_bytes, int roles, int shard_begin = 0, int shard_count = 0);
+
+// The plan of a call whose workspace holds `bytes`: the register-weight
+// products where the call takes them and their buffers fit (a caller of
+// forward_noalloc has a fixed size), else the slot or grouped kernels.
+static PlanKind plan_kind(const grim_moe_layer* L, int tokens, int regime, size_t bytes) {
+    Plan p{};
+    if (use_wreg(L, tokens, regime) && carve(L, tokens, PlanKind::kWreg, nullptr, p) <= bytes) return PlanKind::kWreg;
+    return use_gemv(L, tokens, regime) ? PlanKind::kSlots : PlanKind::kGrouped;
+}
 
 extern "C" int grimoire_moe_forward(void* stream, const grim_moe_layer* L,
                                     const grim_route_params* rp, const uint16_t* shared_gate_w,
@@ -568,7 +704,7 @@ extern "C" int grimoire_moe_forward_noalloc(void* stream, const grim_moe_layer* 
     if (!L || !x || !y) return ferr(GRIM_ERR_ARG, "null layer/x/y");
     if (tokens <= 0) return GRIM_OK;
     Plan p{};
-    const size_t need = carve(L, tokens, use_gemv(L, tokens, regime), nullptr, p);
+    const size_t need = carve(L, tokens, plan_kind(L, tokens, regime, kNoAllocScratchBytes), nullptr, p);
     if (need > kNoAllocScratchBytes) {
         static thread_local char msg[160];
         std::snprintf(msg, sizeof msg,
@@ -618,11 +754,12 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
     const auto& c = L->cfg;
     if (L->has_shared && c.shared_inter != c.inter)
         return ferr(GRIM_ERR_SHAPE, "shared_inter must equal inter");
-    const bool gemv = use_gemv(L, tokens, regime);
+    const PlanKind kind = plan_kind(L, tokens, regime, workspace_bytes);
+    const bool gemv = kind == PlanKind::kSlots;
     Plan p{};
-    const size_t need = carve(L, tokens, gemv, nullptr, p);
+    const size_t need = carve(L, tokens, kind, nullptr, p);
     if (!workspace || workspace_bytes < need) return ferr(GRIM_ERR_WORKSPACE, "workspace too small");
-    carve(L, tokens, gemv, static_cast<char*>(workspace), p);
+    carve(L, tokens, kind, static_cast<char*>(workspace), p);
     if (out_expert) p.rex = out_expert;
     if (out_weight) p.rwt = out_weight;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -777,6 +914,7 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
         return grimoire_moe_down_batched(stream, L, p.rex, p.rwt, p.h, y, tokens);
     }
 
+    if (kind == PlanKind::kWreg) return forward_wreg(st, L, p, x, y, tokens, shared_gate_w);
     if (gv) return forward_gv(st, L, p, x, y, tokens, shared_gate_w, gv_mx, nullptr);
     if (regime == 5 && layer_mx_padded(L))
         return ferr(GRIM_ERR_FORMAT, "regime 5 reads packed MXFP4 rows (K/2 bytes); these are padded");

@@ -1,0 +1,79 @@
+"""The register-weight expert products (grimoire_moe_forward on MXFP4, bf16
+and INT4 batches) against the oracle where their tiles can go wrong: row
+counts around the 16 / 32 / 64 / 128-row blocks, one expert with every token
+and experts with none, K and N with half-filled last segments, scale rows
+whose last window is read early, signed and missing INT4 zero points,
+activations that need their low halves, and a shared expert."""
+import pytest
+import torch
+
+from oracle import oracle as O
+from grimoire_amd import _abi, configs, ops
+from grimoire_amd.weights import Weight
+from tests.helpers import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# x and the weights are exact in bf16; h is a bf16 pair (2^-17 relative per
+# element) and the sums are fp32: 2^-17 plus a few fp32 roundings of sums of
+# a few thousand terms, far below 2e-5.
+TOL = 2e-5
+
+
+def _run(gpu, cfg, seed, zeros=None, fp32_x=False, regime=0):
+    wl = configs.make_workload(cfg, "cpu", seed=seed)
+    L, x = wl.layer, wl.x
+    if zeros is not None:
+        g = torch.Generator().manual_seed(seed)
+        for name in ("gate_up", "down", "shared_gate_up", "shared_down"):
+            w = getattr(L, name)
+            if w is not None:
+                z = torch.randint(0, 16, w.scales.shape, dtype=torch.uint8, generator=g)
+                z[torch.rand(z.shape, generator=g) < zeros] = 0xFF       # signed codes
+                setattr(L, name, Weight(w.fmt, w.N, w.K, w.payload, w.scales, z, w.row_scales))
+    if fp32_x:
+        rows = torch.arange(cfg.T) % 3 == 1
+        x = torch.where(rows[:, None], torch.randn(x.shape, generator=torch.Generator().manual_seed(5)), x).contiguous()
+    # expert 0 takes every token, the last one none
+    bias = torch.zeros(cfg.E)
+    bias[0], bias[-1] = 50.0, -50.0
+    Lg = L.to(gpu)
+    bg = bias.to(gpu)
+    fwd = ops.MoeForward(Lg, cfg.T, configs.route_params(cfg, bg), regime)
+    xg = x.to(gpu)
+    y = torch.full((cfg.T, cfg.H), float("nan"), device=gpu)
+    oe = torch.empty(cfg.T, cfg.K, dtype=torch.int32, device=gpu)
+    ow = torch.empty(cfg.T, cfg.K, device=gpu)
+    fwd(xg, y, oe, ow)
+    torch.cuda.synchronize()
+    oe, ow = oe.cpu(), ow.cpu()
+    assert (oe[:, 0] == 0).all() and (oe != cfg.E - 1).all()
+    gate = None
+    if L.has_shared and L.shared_gate_w is not None:
+        gw = (L.shared_gate_w.to(torch.int32) << 16).view(torch.float32)
+        gate = torch.sigmoid(x.double() @ gw.double()).float().contiguous()
+    want = O.moe_forward(L.struct(), oe, ow, gate, x)
+    err = rel_l2(y.cpu(), want)
+    assert err <= TOL, err
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 64, 65, 128, 129, 193])
+@pytest.mark.parametrize("fmt", ["mxfp4", "bf16"])
+def test_row_blocks(gpu, fmt, T):
+    print(f"wreg {fmt} T={T}", flush=True)
+    _run(gpu, configs.Config("t", T, 576, 6, 3, 704, fmt, shared=T % 2 == 1, shared_gate=T % 4 == 1), seed=T, regime=2)
+
+
+@pytest.mark.parametrize("H,I", [(512, 576), (2112, 512), (2880, 1024), (4096, 640)])
+def test_mxfp4_scale_windows(gpu, H, I):
+    """Scale rows of 16, 18, 20, 66, 90 and 128 bytes: whole, early and
+    several chunks of windows."""
+    print(f"wreg mxfp4 H={H} I={I}", flush=True)
+    _run(gpu, configs.Config("t", 40, H, 5, 2, I, "mxfp4"), seed=H, regime=2)
+
+
+@pytest.mark.parametrize("H,I", [(512, 640), (2176, 512), (2688, 896)])
+@pytest.mark.parametrize("zeros,fp32_x", [(None, False), (0.5, False), (0.0, True), (None, True)])
+def test_int4(gpu, H, I, zeros, fp32_x):
+    print(f"wreg int4 H={H} I={I} zeros={zeros} fp32_x={fp32_x}", flush=True)
+    _run(gpu, configs.Config("t", 35, H, 36, 2, I, "int4", shared=True), seed=H, zeros=zeros, fp32_x=fp32_x)
