@@ -171,16 +171,27 @@ bool wreg_ok(const grim_moe_layer* L, int T) {
 
 // ... and the call takes them: MXFP4 and bf16 experts wherever the grouped
 // GEMM would run (1000 tokens of 128 MXFP4 experts, H = I = 2880: 1300 ->
-// 660 us a layer; 150 tokens of 64 bf16 experts: 299 -> 231 us); INT4 experts
-// above 64 routes (fewer stay with the slot kernels) up to the two routes per
-// expert that INT4 batches are taken for, where the vector-ALU grouped GEMV
-// ran (20 tokens x top-8 of 128, H 2048, I 768: 304 -> 87 us).
+// 660 us a layer; 150 tokens of 64 bf16 experts: 299 -> 225 us).  INT4
+// experts, up to the two routes per expert that INT4 batches are taken for:
+// above 64 routes always (the vector-ALU grouped GEMV otherwise: 20 tokens x
+// top-8 of 128, H 2048, I 768: 304 -> 76 us), below when the bytes that the
+// slot kernels read, every route its expert, cost more than the three extra
+// launches: 16 tokens x top-4, H 2048, I 1024 (209 MB) 107 -> 54 us; 12 x
+// top-2, I 768 (58 MB) 34.4 / 34.6; 9 x top-2, H 1024, I 512 (15 MB) 21 / 28.
+// Up to 8 tokens the slot kernels are the faster three-launch decode: 8 x
+// top-4, H 4096, I 2048 (410 MB) 117 -> 95 us; 4 x top-4 of them (205 MB)
+// 65 / 64; 8 x top-8, H 2048, I 768 (151 MB) 56 / 57.
 bool use_wreg(const grim_moe_layer* L, int T, int regime) {
     const int64_t R = int64_t(T) * L->cfg.top_k;
     const int f = L->gate_up.fmt;
     if (!wreg_ok(L, T)) return false;
-    if (f == GRIM_FMT_INT4 || f == GRIM_FMT_INT4_F16)
-        return regime == 0 && R > 64 && R <= 2 * int64_t(L->cfg.num_experts);
+    if (f == GRIM_FMT_INT4 || f == GRIM_FMT_INT4_F16) {
+        const int64_t expert = 2 * L->cfg.inter * L->gate_up.row_bytes + L->cfg.hidden * L->down.row_bytes;
+        const int64_t slot_bytes = (R + (L->has_shared ? T : 0)) * expert;
+        if (regime != 0 || T <= 1) return false;
+        return R > 64 ? R <= 2 * int64_t(L->cfg.num_experts)
+                      : slot_bytes >= (T > kDecodeMaxTokens ? int64_t(48) << 20 : int64_t(192) << 20);
+    }
     if (regime == 2) return true;
     return regime == 0 && !use_gemv(L, T, 0) &&
            !(f == GRIM_FMT_MXFP4 && R <= 2 * int64_t(L->cfg.num_experts) && gv_ok(L));
@@ -526,10 +537,18 @@ static int forward_gv(hipStream_t st, const grim_moe_layer* L, const Plan& p, co
 // gate_up + SwiGLU (h as a bf16 pair per route) -> down (fp32 rows per
 // route) -> combine.
 static int forward_wreg(hipStream_t st, const grim_moe_layer* L, const Plan& p, const float* x, float* y,
-                        int tokens, const uint16_t* shared_gate_w) {
+                        int tokens, const uint16_t* shared_gate_w, const TopkArgs* route) {
     const auto& c = L->cfg;
     const int E = c.num_experts, K = c.top_k, H = c.hidden, I = c.inter, f = L->gate_up.fmt;
     const bool sh = L->has_shared;
+    // small batches: the top-k (when `route` leaves it to this path), the
+    // dispatch and the x planes in one launch
+    const bool one = wreg_one_dispatch(tokens, K, E);
+    TopkArgs tk{};
+    if (route) tk = *route;
+    tk.T = tokens;
+    tk.K = K;
+    tk.out_e = p.rex;
     DispatchArgs da{};
     da.ids = p.rex;
     da.T = tokens;
@@ -541,9 +560,9 @@ static int forward_wreg(hipStream_t st, const grim_moe_layer* L, const Plan& p, 
     da.perm_token = p.wr_perm;
     da.workspace = p.disp_ws;
     da.lists = TileLists{{p.wr_tiles[0], p.wr_tiles[1]}, {wreg_mc(f, true), wreg_mc(f, false)}, p.wr_live};
-    hipError_t e = dispatch_launch(st, da);
+    hipError_t e = one ? hipSuccess : dispatch_launch(st, da);
     if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
-    e = wreg_format_launch(st, f, x, tokens, H, p.wr_x, p.wr_lo);
+    e = wreg_route_launch(st, f, x, H, p.wr_x, p.wr_lo, tk, one ? &da : nullptr, route != nullptr);
     if (e == hipSuccess && sh && shared_gate_w) e = rowdot_sigmoid_launch(st, x, shared_gate_w, p.gate, tokens, H);
     if (e != hipSuccess) return ferr(int(e), hipGetErrorString(e));
     WregArgs g{};
@@ -880,6 +899,8 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
         }
         return forward_gv(st, L, p, x, y, tokens, shared_gate_w, true, &tka);
     }
+    if (kind == PlanKind::kWreg && !shard && !deferred && wreg_one_dispatch(tokens, K, E) && wreg_one_topk(tokens))
+        return forward_wreg(st, L, p, x, y, tokens, shared_gate_w, &tka);
     if (deferred) {
         // the top-k finishes the split router's sum as it loads
         tka.part1 = p.logits2;
@@ -914,7 +935,7 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
         return grimoire_moe_down_batched(stream, L, p.rex, p.rwt, p.h, y, tokens);
     }
 
-    if (kind == PlanKind::kWreg) return forward_wreg(st, L, p, x, y, tokens, shared_gate_w);
+    if (kind == PlanKind::kWreg) return forward_wreg(st, L, p, x, y, tokens, shared_gate_w, nullptr);
     if (gv) return forward_gv(st, L, p, x, y, tokens, shared_gate_w, gv_mx, nullptr);
     if (regime == 5 && layer_mx_padded(L))
         return ferr(GRIM_ERR_FORMAT, "regime 5 reads packed MXFP4 rows (K/2 bytes); these are padded");

@@ -43,6 +43,9 @@
 // 257 us.
 #include "gemm_wreg.hpp"
 
+#include "dispatch_one.hpp"
+#include "topk.hpp"
+
 #include <algorithm>
 #include <utility>
 
@@ -551,15 +554,15 @@ __global__ __launch_bounds__(kWregThreads, WregFmt<F>::WG) void grouped_wreg_ker
     }
 }
 
-// x rows as bf16 planes in the order the weights decode to; K padded with
-// zeros.  One work-group per row.
+// One x row as bf16 planes in the order the weights decode to, K padded
+// with zeros.
 template <bool INT4>
-__global__ __launch_bounds__(256) void wreg_format_kernel(const float* __restrict__ x, int H, int Kp,
-                                                          uint16_t* __restrict__ dst, int32_t* __restrict__ lo) {
-    const float* xr = x + int64_t(blockIdx.x) * H;
-    uint16_t* d = dst + int64_t(blockIdx.x) * (INT4 ? 2 : 1) * Kp;
+__device__ __forceinline__ void wreg_format_row(const float* __restrict__ x, int t, int H, int Kp,
+                                                uint16_t* __restrict__ dst, int32_t* __restrict__ lo) {
+    const float* xr = x + int64_t(t) * H;
+    uint16_t* d = dst + int64_t(t) * (INT4 ? 2 : 1) * Kp;
     int any = 0;
-    for (int k = threadIdx.x * 8; k < Kp; k += 256 * 8) {
+    for (int k = threadIdx.x * 8; k < Kp; k += blockDim.x * 8) {
         float v[8];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -585,8 +588,50 @@ __global__ __launch_bounds__(256) void wreg_format_kernel(const float* __restric
     }
     if constexpr (INT4) {
         const int r = __syncthreads_or(any);
-        if (threadIdx.x == 0) lo[blockIdx.x] = r ? 1 : 0;
+        if (threadIdx.x == 0) lo[t] = r ? 1 : 0;
     }
+}
+
+// Work-group 0 (`route`): the top-k of up to 16 tokens, one wave each
+// (topk_kernel's code, so the same bits; more tokens would share one CU),
+// and the dispatch; the other work-groups format one token row each
+// meanwhile.  One launch of 9.0 us for 16 tokens x top-4 where top-k, four
+// dispatch launches and the formatting took 27.
+template <bool INT4>
+__global__ __launch_bounds__(kOneThreads) void wreg_route_kernel(const float* x, int H, int Kp, uint16_t* dst,
+                                                                 int32_t* lo, TopkArgs tk, OneArgs oa, int route,
+                                                                 int topk) {
+    struct TopkLds {
+        float gsel[kOneWaves][512];
+        float gscore[kOneWaves][64];
+        int32_t e[kOneWaves][16];
+        float w[kOneWaves][16];
+    };
+    __shared__ union { OneLds one; TopkLds tk; } lds;
+    if (int(blockIdx.x) >= route) {
+        wreg_format_row<INT4>(x, int(blockIdx.x) - route, H, Kp, dst, lo);
+        return;
+    }
+    if (!topk) {
+        dispatch_one_block(oa, lds.one, [&](int r) { return tk.out_e[r]; });
+        return;
+    }
+    const int wv = threadIdx.x / kWave, R = tk.T * tk.K;
+    if (wv < tk.T)
+        topk_wave(tk.logits + int64_t(wv) * tk.E, tk.E, tk.K, tk.mode, tk.normalize, tk.scaling, tk.bias16, tk.bias32,
+                  tk.n_group, tk.topk_group, lds.tk.e[wv], lds.tk.w[wv], lds.tk.gsel[wv], lds.tk.gscore[wv]);
+    __syncthreads();
+    // (at most 16 tokens x 16 picks: one route per thread of the first waves)
+    const int r = threadIdx.x;
+    int pe = -1;
+    if (r < R) {
+        pe = lds.tk.e[r / tk.K][r % tk.K];
+        tk.out_e[r] = pe;
+        tk.out_w[r] = lds.tk.w[r / tk.K][r % tk.K];
+    }
+    __syncthreads();
+    // with R <= 1024 the dispatch asks each thread for its own route only
+    dispatch_one_block(oa, lds.one, [&](int) { return pe; });
 }
 
 static bool is_int4(int fmt) { return fmt == GRIM_FMT_INT4 || fmt == GRIM_FMT_INT4_F16; }
@@ -617,13 +662,24 @@ bool wreg_weight_ok(const grim_quant_weight& w, int rows_per_expert, int K) {
     return false;
 }
 
-hipError_t wreg_format_launch(hipStream_t st, int fmt, const float* x, int T, int H, uint16_t* dst, int32_t* lo) {
-    if (T <= 0) return hipSuccess;
-    const int Kp = wreg_kpad(fmt, H);
+bool wreg_one_dispatch(int T, int K, int E) { return int64_t(T) * K <= kOneMaxRoutes && E <= kOneMaxE; }
+bool wreg_one_topk(int T) { return T <= kOneWaves; }
+
+hipError_t wreg_route_launch(hipStream_t st, int fmt, const float* x, int H, uint16_t* dst, int32_t* lo,
+                             const TopkArgs& tk, const DispatchArgs* d, bool topk) {
+    if (tk.T <= 0) return hipSuccess;
+    if (d && !wreg_one_dispatch(d->T, d->K, d->E)) return hipErrorInvalidValue;
+    if (topk && (!d || !wreg_one_topk(tk.T) || tk.K > 16 || tk.E > 512 || tk.part1)) return hipErrorInvalidValue;
+    OneArgs oa{};
+    if (d)
+        oa = OneArgs{d->T * d->K, d->E, d->K, d->counts, d->offsets, d->inverse, d->perm_token, d->lists,
+                     nullptr, nullptr, 0, 0, nullptr};
+    const int Kp = wreg_kpad(fmt, H), route = d ? 1 : 0;
+    const dim3 grid(tk.T + route), block(d ? kOneThreads : 256);
     if (is_int4(fmt))
-        hipLaunchKernelGGL(wreg_format_kernel<true>, dim3(T), dim3(256), 0, st, x, H, Kp, dst, lo);
+        hipLaunchKernelGGL(wreg_route_kernel<true>, grid, block, 0, st, x, H, Kp, dst, lo, tk, oa, route, int(topk));
     else
-        hipLaunchKernelGGL(wreg_format_kernel<false>, dim3(T), dim3(256), 0, st, x, H, Kp, dst, lo);
+        hipLaunchKernelGGL(wreg_route_kernel<false>, grid, block, 0, st, x, H, Kp, dst, lo, tk, oa, route, int(topk));
     return hipGetLastError();
 }
 

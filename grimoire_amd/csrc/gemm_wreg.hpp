@@ -4,6 +4,7 @@
 
 #include "common.hpp"
 #include "dispatch.hpp"
+#include "router.hpp"
 
 namespace grim {
 
@@ -40,8 +41,15 @@ int wreg_kpad(int fmt, int K);
 // Activation planes of gate_up: INT4 experts split fp32 x exactly in two
 // bf16 halves, the others round x to bf16.
 int wreg_x_planes(int fmt);
-// x fp32 [T][H] -> bf16 rows [T][planes][wreg_kpad] (+ per row lo != 0)
-hipError_t wreg_format_launch(hipStream_t st, int fmt, const float* x, int T, int H, uint16_t* dst, int32_t* lo);
+// x fp32 [T][H] -> bf16 rows [T][planes][wreg_kpad] (+ per row lo != 0), and
+// in the same launch the dispatch of the routes in tk.out_e (its first
+// work-group) with the top-k before it when `topk` -- where
+// wreg_one_dispatch / wreg_one_topk hold; otherwise d is null and both ran
+// before.
+bool wreg_one_dispatch(int T, int K, int E);
+bool wreg_one_topk(int T);
+hipError_t wreg_route_launch(hipStream_t st, int fmt, const float* x, int H, uint16_t* dst, int32_t* lo,
+                             const TopkArgs& tk, const DispatchArgs* d, bool topk);
 hipError_t wreg_launch(hipStream_t st, int fmt, const WregArgs& a, bool gate_up);
 
 }  // namespace grim
