@@ -7,7 +7,6 @@
 #include "topk.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace grim {
 
@@ -496,6 +495,167 @@ __global__ __launch_bounds__(256) void router_bf16x3(const float* __restrict__ W
     }
 }
 
+// The three-limb products for a few dozen to a thousand tokens: 32 tokens x 32
+// experts per work-group, K split over its 16 waves.  At these sizes the
+// tiles above leave most CUs idle and walk K alone (201 tokens, E = 512, H =
+// 2048: 32 work-groups, 42 us; 150 tokens, E = 64: 3, 40 us), bound by the
+// latency of their K tiles.  Here a wave takes a sixteenth of K: operands
+// straight from global memory into the registers the matrix instruction
+// reads (K permuted so that the four lanes of a row read 64 consecutive
+// bytes), no LDS until the 16 partial sums are added in wave order.  x that is all bf16 values in a unit runs only the
+// three products of its one limb (the others are exact zeros).
+//
+// K is cut into two halves of 16 waves' parts each, whatever the launch: the
+// halves' sums a and b are added as (a + b) + bias.  With few tiles the
+// halves run as work-groups of their own (SPLIT: a to logits, b to part1,
+// finished by the top-k), else one after the other.  The tile (NJ blocks of
+// 16 experts) does not change the sums either, so the standalone and the
+// forward's logits are the same bits.  A CU takes its operands in at ~50
+// GB/s here (with the products taken out 38 of 41 us are left at 201 tokens,
+// E = 256, H = 7168), so the tile is the one that spreads over the most CUs
+// in one round.  150 tokens, E = 64, H = 2048: 40 -> 10 us (split); 201, E =
+// 512: 42 -> 19; 1000, E = 128, H = 2880: 48 -> 31 against the 128 x 128
+// tiles with their W image.  Errors against 64 bits 4.9e-7 -> 1.1e-7.
+constexpr int kRkWaves = 16, kRkUnit = 32;
+typedef float f32x4r __attribute__((ext_vector_type(4)));
+template <int NJ, bool SPLIT>
+__global__ __launch_bounds__(kRkWaves * 64) void router_bf16x3_k16(const float* __restrict__ W,
+                                                                   const float* __restrict__ x,
+                                                                   const float* __restrict__ bias,
+                                                                   float* __restrict__ logits,
+                                                                   float* __restrict__ part1, int T, int E, int H) {
+    constexpr int MI = 2, NS = 2;
+    __shared__ float part[kRkWaves][4 * MI * NJ][64];
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = blockIdx.x * (16 * MI), e0 = blockIdx.y * (16 * NJ);
+    const float *xr[MI], *wr[NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) xr[i] = x + int64_t(min(t0 + 16 * i + c, T - 1)) * H + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) wr[j] = W + int64_t(min(e0 + 16 * j + c, E - 1)) * H + 4 * g;
+    const int nu = H / kRkUnit, nh = (nu + 1) / 2, per = (nh + kRkWaves - 1) / kRkWaves;
+    // thread's output: wave (i, j, v) adds the waves' sums of acc[i][j][v], token 16 i + 4 g + v, expert 16 j + c
+    const int t = t0 + 16 * (wave / (4 * NJ)) + 4 * g + (wave & 3), e = e0 + 16 * ((wave >> 2) % NJ) + c;
+    const bool mine = wave < 4 * MI * NJ && t < T && e < E;
+    f32x4n rx[NS][MI][2], rw[NS][NJ][2];
+    // unit u into set s (past the last unit the last again, never used)
+    auto load = [&](int s, int u) __attribute__((always_inline)) {
+        const int k = min(u, nu - 1) * kRkUnit;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) rw[s][j][q] = *reinterpret_cast<const f32x4n*>(wr[j] + k + 16 * q);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) rx[s][i][q] = *reinterpret_cast<const f32x4n*>(xr[i] + k + 16 * q);
+        }
+    };
+    auto limbs = [](const f32x4n (&v)[2], bf16x8r (&out)[3]) __attribute__((always_inline)) {
+        uint32_t b[3][4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            uint32_t o[3][2];
+            split3(v[q], o);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) { b[p][2 * q] = o[p][0]; b[p][2 * q + 1] = o[p][1]; }
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p) __builtin_memcpy(&out[p], b[p], 16);
+    };
+    f32x4r acc[MI][NJ];
+    auto mul = [&](const f32x4n (&vx)[MI][2], const f32x4n (&vw)[NJ][2]) __attribute__((always_inline)) {
+        uint32_t low = 0;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) low |= __float_as_uint(vx[i][q][k]);
+        const bool full = __ballot((low & 0xFFFFu) != 0) != 0;   // uniform
+        bf16x8r b[NJ][3];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) limbs(vw[j], b[j]);
+        // smallest products first: mm, lh, hl, mh, hm, hh
+        constexpr int pa[6] = {1, 2, 0, 1, 0, 0}, pb[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            if (full) {
+                bf16x8r a[3];
+                limbs(vx[i], a);
+#pragma unroll
+                for (int p = 0; p < 6; ++p)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa[p]], b[j][pb[p]], acc[i][j], 0, 0, 0);
+            } else {
+                uint32_t w[4];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                        w[2 * q + k] = __builtin_amdgcn_perm(__float_as_uint(vx[i][q][2 * k + 1]),
+                                                             __float_as_uint(vx[i][q][2 * k]), 0x07060302u);
+                bf16x8r a;
+                __builtin_memcpy(&a, w, 16);
+#pragma unroll
+                for (int p = 2; p >= 0; --p)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j][p], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int z = 0; z < (SPLIT ? 1 : 2); ++z) {
+        const int half = SPLIT ? int(blockIdx.z) : z;
+        const int u0 = half * nh + wave * per, u1 = min(min(u0 + per, nh * (half + 1)), nu);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4r{0.f, 0.f, 0.f, 0.f};
+        if (u0 < u1) {   // uniform
+#pragma unroll
+            for (int s = 0; s < NS; ++s) load(s, u0 + s);
+            for (int u = u0; u < u1; u += NS) {
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    if (u + s < u1) mul(rx[s], rw[s]);
+                    load(s, u + s + NS);
+                }
+            }
+        }
+        if (z) __syncthreads();   // the first half's sums have been read
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) part[wave][(i * NJ + j) * 4 + v][lane] = acc[i][j][v];
+        __syncthreads();
+        if (wave < 4 * MI * NJ) {
+            float s = part[0][wave][lane];
+#pragma unroll
+            for (int w = 1; w < kRkWaves; ++w) s += part[w][wave][lane];
+            sum[z] = s;
+        }
+    }
+    if (!mine) return;
+    if constexpr (SPLIT) {
+        (blockIdx.z ? part1 : logits)[int64_t(t) * E + e] = sum[0];
+    } else {
+        const float s = sum[0] + sum[1];
+        logits[int64_t(t) * E + e] = bias ? s + bias[e] : s;
+    }
+}
+
+// Work-groups of the k16 router at NJ blocks of 16 experts.
+static int64_t rk_groups(int T, int E, int nj) { return int64_t((T + 31) / 32) * ((E + 16 * nj - 1) / (16 * nj)); }
+// One round of tiles over the 256 CUs (512 tokens x 512 experts, H = 2048,
+// exactly one round of the wider ones: 24 us, the 128 x 128 tiles 31; two
+// rounds, 1000 tokens: 37 against 32).
+static bool rk_ok(int T, int E, int H) { return H % kRkUnit == 0 && rk_groups(T, E, 2) <= 256; }
+
 // The same three-limb products on 128 x 128 tiles with K split in two
 // halves (grid z).  At T = 4096, E = 512 a 64 x 64 tile per work-group reads
 // its 64 x rows and 64 W rows over the whole K (2 MB per CU); a 128 x 128
@@ -814,6 +974,16 @@ hipError_t router_logits_launch(hipStream_t st, const float* W, const float* x,
     } else if (T <= 32 && H % 4 == 0) {
         dim3 grid(E, (T + kRouterTok - 1) / kRouterTok);
         hipLaunchKernelGGL(router_gemv, grid, dim3(256), 0, st, W, x, bias, logits, T, E, H);
+    } else if (rk_ok(T, E, H)) {
+        const int nj = rk_groups(T, E, 1) <= 256 ? 1 : 2;
+        const bool split = part1 && deferred && rk_groups(T, E, nj) <= 128;
+        const dim3 grid((T + 31) / 32, (E + 16 * nj - 1) / (16 * nj), split ? 2 : 1), block(kRkWaves * 64);
+        if (split) hipLaunchKernelGGL((router_bf16x3_k16<1, true>), grid, block, 0, st, W, x, bias, logits, part1, T, E, H);
+        else if (nj == 1)
+            hipLaunchKernelGGL((router_bf16x3_k16<1, false>), grid, block, 0, st, W, x, bias, logits, part1, T, E, H);
+        else
+            hipLaunchKernelGGL((router_bf16x3_k16<2, false>), grid, block, 0, st, W, x, bias, logits, part1, T, E, H);
+        if (split) *deferred = 1;
     } else if (H % (2 * kR3BK) == 0 && H >= 2 * kR3BK * kRsPre && T >= 256) {
         // split K.  With part1 and deferred: the halves store a (logits) and
         // b (part1), and the caller finishes (a + b) + bias (the top-k's
