@@ -33,6 +33,7 @@ struct DecodeArgs {
     int H, I, K, E, M;
     // plan (decode_plan)
     int lpr_gu, lpr_dn, gu_rb, dn_rb;
+    int gu_nb, dn_nb;         // row blocks per gate_up / down item (slot kernels; wave-centric ones: 1)
     int NR, NG, ND;
     int fmt_h;                // gate_up writes hf, down stages hf (else plain h)
     int route_topk;           // gate_up items compute the top-k from logits (and store rex/rwt)
@@ -80,6 +81,9 @@ __host__ __device__ constexpr int fmt_words(int n) { return (n + n / 8 + 3) & ~3
 // (32-element chunks, H = 32 * C): hi plane [H/2], lo plane [H/2], then
 // (sum, lo-nonzero flag) per chunk, padded to 16 bytes.
 __host__ __device__ constexpr int xf_words(int H) { return (H + 2 * (H / 32) + 3) & ~3; }
+
+// Row blocks per gate_up item, at most (their h rows wait in LDS).
+constexpr int kGuMaxNB = 8;
 
 constexpr int kRoleRouter = 1, kRoleGateUp = 2, kRoleDown = 4;
 

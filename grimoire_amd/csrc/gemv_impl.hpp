@@ -512,32 +512,84 @@ __device__ __forceinline__ void router_item(const DecodeArgs& a, int b) {
         a.logits[int64_t(threadIdx.x) * a.E + e] = a.rbias ? s + a.rbias[e] : s;
 }
 
-// gate_up rows of one (token, slot, row block): RU (gate, up) row pairs per
-// lane group, one chunk of the next iteration in flight while this one is
-// multiplied.
-template <int F, int LPR, bool LO>
-__device__ __forceinline__ void gate_up_rows(const WView& v, int64_t gbase, int i0, int I, int C,
-                                             int sub, const uint32_t* act, int n,
-                                             Pre (&cur)[2][kRuGU], float* ga, float* ua) {
-    for (int c = sub; c < C; c += LPR) {
-        Pre nxt[2][kRuGU];
-        const int cn = c + LPR;
-        if (cn < C) {
+// gate_up rows of nb row blocks of one (token, slot): RU (gate, up) row pairs
+// per lane group and block, the blocks' chunks one stream with the next
+// chunk in flight while this one is multiplied.  cur holds the first; done
+// takes each block's sums.
+template <int F, int LPR, bool LO, class Done>
+__device__ __forceinline__ void gate_up_rows(const WView& v, int64_t gbase, int i0, int rstep, int nb, int I,
+                                             int C, int sub, const uint32_t* act, int n,
+                                             Pre (&cur)[2][kRuGU], Done done) {
+    if (nb == 1) {
+        // (its own loop: one token's items end with their only block, and
+        // the stream's bookkeeping costs them 3%)
+        float ga[kRuGU], ua[kRuGU];
+#pragma unroll
+        for (int r = 0; r < kRuGU; ++r) ga[r] = ua[r] = 0.0f;
+        for (int c = sub; c < C; c += LPR) {
+            Pre nxt[2][kRuGU];
+            const int cn = c + LPR;
+            if (cn < C) {
+#pragma unroll
+                for (int r = 0; r < kRuGU; ++r) {
+                    const int i = i0 + r < I ? i0 + r : I - 1;
+                    prefetch<F>(v, gbase + i, cn, nxt[0][r]);
+                    prefetch<F>(v, gbase + I + i, cn, nxt[1][r]);
+                }
+            }
+            XChunk<F, LO> x;
+            load_x<F, LO>(act, n, c, x);
 #pragma unroll
             for (int r = 0; r < kRuGU; ++r) {
-                const int i = i0 + r < I ? i0 + r : I - 1;
-                prefetch<F>(v, gbase + i, cn, nxt[0][r]);
-                prefetch<F>(v, gbase + I + i, cn, nxt[1][r]);
+                ga[r] += dot_chunk<F, LO>(cur[0][r], x);
+                ua[r] += dot_chunk<F, LO>(cur[1][r], x);
+            }
+            if (cn < C) {
+#pragma unroll
+                for (int r = 0; r < kRuGU; ++r) { cur[0][r] = nxt[0][r]; cur[1][r] = nxt[1][r]; }
             }
         }
-        XChunk<F, LO> x;
-        load_x<F, LO>(act, n, c, x);
+        done(0, ga, ua);
+        return;
+    }
+    const int nc = (C + LPR - 1) / LPR;   // chunk iterations per block
+    float ga[kRuGU], ua[kRuGU];
 #pragma unroll
-        for (int r = 0; r < kRuGU; ++r) {
-            ga[r] += dot_chunk<F, LO>(cur[0][r], x);
-            ua[r] += dot_chunk<F, LO>(cur[1][r], x);
+    for (int r = 0; r < kRuGU; ++r) ga[r] = ua[r] = 0.0f;
+    int blk = 0, ci = 0;
+    for (int it = nb * nc; it > 0; --it) {
+        Pre nxt[2][kRuGU];
+        const bool last = ci + 1 == nc;                  // of this block (uniform)
+        const int cn = sub + (last ? 0 : (ci + 1) * LPR);
+        if (it > 1) {
+            const int in = i0 + (last ? blk + 1 : blk) * rstep, cc = cn < C ? cn : C - 1;
+#pragma unroll
+            for (int r = 0; r < kRuGU; ++r) {
+                const int i = in + r < I ? in + r : I - 1;
+                prefetch<F>(v, gbase + i, cc, nxt[0][r]);
+                prefetch<F>(v, gbase + I + i, cc, nxt[1][r]);
+            }
         }
-        if (cn < C) {
+        const int c = sub + ci * LPR;
+        if (c < C) {
+            XChunk<F, LO> x;
+            load_x<F, LO>(act, n, c, x);
+#pragma unroll
+            for (int r = 0; r < kRuGU; ++r) {
+                ga[r] += dot_chunk<F, LO>(cur[0][r], x);
+                ua[r] += dot_chunk<F, LO>(cur[1][r], x);
+            }
+        }
+        if (last) {
+            done(blk, ga, ua);
+#pragma unroll
+            for (int r = 0; r < kRuGU; ++r) ga[r] = ua[r] = 0.0f;
+            ++blk;
+            ci = 0;
+        } else {
+            ++ci;
+        }
+        if (it > 1) {
 #pragma unroll
             for (int r = 0; r < kRuGU; ++r) { cur[0][r] = nxt[0][r]; cur[1][r] = nxt[1][r]; }
         }
@@ -552,9 +604,11 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
     const int H = a.H, I = a.I, K = a.K;
     const int KS = K + (SH ? 1 : 0);
     const int C = H / Chunk<F>::CH;
-    const int t = j / (KS * a.gu_rb);
-    const int slot = (j / a.gu_rb) % KS;
-    const int rb = j % a.gu_rb;
+    const int groups = (a.gu_rb + a.gu_nb - 1) / a.gu_nb;   // of gu_nb row blocks
+    const int t = j / (KS * groups);
+    const int slot = (j / groups) % KS;
+    const int rb = j % groups * a.gu_nb;                    // first row block
+    const int nb = min(a.gu_nb, a.gu_rb - rb);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int sub = lane % LPR;
@@ -601,12 +655,9 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
     // (3) this item's weights, all requested before anything waits on them
     const WView v = (SH && shr) ? a.sgu : a.gu;
     if (!active) gbase = 0;   // rows of expert 0 are read and discarded
-    float ga[RU], ua[RU];
     Pre cur[2][RU];
 #pragma unroll
     for (int r = 0; r < RU; ++r) {
-        ga[r] = 0.0f;
-        ua[r] = 0.0f;
         const int i = i0 + r < I ? i0 + r : I - 1;
         const int c = sub < C ? sub : 0;
         prefetch<F>(v, gbase + i, c, cur[0][r]);
@@ -615,33 +666,39 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
     // (4) the activations into LDS while the weights are in flight
     const bool lo_pass = x_store<F>(xr, H, lds);
     GRIM_TS(a, 1, 2);
+    __shared__ float hrow[kGuMaxNB * kGemvWaves * kWave / 8 * RU];   // this item's rows (fmt_h)
+    auto done = [&](int blk, const float (&ga)[RU], const float (&ua)[RU]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RU; ++r) {
+            const float g = group_sum<LPR>(ga[r]);
+            const float u = group_sum<LPR>(ua[r]);
+            const int i = i0 + blk * RB + r;
+            const float hv = active ? silu(g) * u : 0.0f;
+            if (a.fmt_h) {
+                if (sub == 0) hrow[blk * RB + (wave * GPW + lane / LPR) * RU + r] = i < I ? hv : 0.0f;
+            } else if (sub == 0 && i < I) {
+                ht[i] = hv;
+            }
+        }
+    };
     if (active) {
-        if (lo_pass) gate_up_rows<F, LPR, true>(v, gbase, i0, I, C, sub, lds, H, cur, ga, ua);
-        else gate_up_rows<F, LPR, false>(v, gbase, i0, I, C, sub, lds, H, cur, ga, ua);
+        if (lo_pass) gate_up_rows<F, LPR, true>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
+        else gate_up_rows<F, LPR, false>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
+    } else {
+        const float zero[RU] = {};
+        for (int blk = 0; blk < nb; ++blk) done(blk, zero, zero);
     }
     GRIM_TS(a, 1, 3);
-    __shared__ float hrow[kGemvWaves * kWave / 8 * RU];   // this item's RB rows (fmt_h)
-#pragma unroll
-    for (int r = 0; r < RU; ++r) {
-        const float g = group_sum<LPR>(ga[r]);
-        const float u = group_sum<LPR>(ua[r]);
-        const int i = i0 + r;
-        const float hv = active ? silu(g) * u : 0.0f;
-        if (a.fmt_h) {
-            if (sub == 0) hrow[(wave * GPW + lane / LPR) * RU + r] = i < I ? hv : 0.0f;
-        } else if (sub == 0 && i < I) {
-            ht[i] = hv;
-        }
-    }
     if (a.fmt_h) {
-        // the RB rows as RB / 8 formatted groups of the token's h vector
+        // the rows as groups of eight formatted elements of the token's h vector
         __syncthreads();
         const int n = KS * I;
-        const int i8 = rb * RB + 8 * int(threadIdx.x);
-        if (int(threadIdx.x) < RB / 8 && i8 < I) {
+        for (int k8 = threadIdx.x; k8 < nb * RB / 8; k8 += kGemvThreads) {
+            const int i8 = rb * RB + 8 * k8;
+            if (i8 >= I) continue;
             float hv[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) hv[k] = hrow[8 * threadIdx.x + k];
+            for (int k = 0; k < 8; ++k) hv[k] = hrow[8 * k8 + k];
             put_group_fmt<F>(a.hf + int64_t(t) * fmt_words(n), n, (slot * I + i8) / 8, hv);
         }
     }
@@ -662,30 +719,65 @@ constexpr int kDnBatch = 3;
 
 template <int F, int LPR>
 __device__ __forceinline__ void down_issue(const DecodeArgs& a, const bool* pvalid,
-                                           const bool* pshared, const int64_t* wrow, int C,
-                                           int c0, Pre (&w)[kDnBatch][kPairsDN]) {
+                                           const bool* pshared, const int64_t* wbase, const int* prow, int o0,
+                                           int C, int c0, Pre (&w)[kDnBatch][kPairsDN]) {
     // clamped addresses instead of branches around the loads (chunks past
-    // the row end and invalid pairs are loaded and never used)
+    // the row end, rows past the last and invalid pairs are loaded and never
+    // used)
 #pragma unroll
     for (int b = 0; b < kDnBatch; ++b) {
         const int c = c0 + b * LPR;
         const int cc = c < C ? c : C - 1;
 #pragma unroll
         for (int q = 0; q < kPairsDN; ++q)
-            prefetch<F>(pshared[q] ? a.sdn : a.dn, pvalid[q] ? wrow[q] : 0, cc, w[b][q]);
+            prefetch<F>(pshared[q] ? a.sdn : a.dn, pvalid[q] ? wbase[q] + min(o0 + prow[q], a.H - 1) : 0, cc, w[b][q]);
     }
 }
 
-template <int F, int LPR, bool LO>
+// nb row blocks of rstep rows from row o0, their chunk batches one stream
+// with the next batch in flight; w holds the first.  done takes each
+// block's sums.
+template <int F, int LPR, bool LO, class Done>
 __device__ __forceinline__ void down_rows(const DecodeArgs& a, const int* pslot, const bool* pvalid,
-                                          const bool* pshared, const int64_t* wrow, int C, int sub,
-                                          const uint32_t* act, int n,
-                                          Pre (&w)[kDnBatch][kPairsDN], float* acc) {
-    for (int c0 = sub; c0 < C; c0 += kDnBatch * LPR) {
-        if (c0 != sub) down_issue<F, LPR>(a, pvalid, pshared, wrow, C, c0, w);
+                                          const bool* pshared, const int64_t* wbase, const int* prow, int o0,
+                                          int rstep, int nb, int C, int sub, const uint32_t* act, int n,
+                                          Pre (&w)[kDnBatch][kPairsDN], Done done) {
+    if (nb == 1) {   // (as in gate_up_rows)
+        float acc[kPairsDN];
+#pragma unroll
+        for (int q = 0; q < kPairsDN; ++q) acc[q] = 0.0f;
+        for (int c0 = sub; c0 < C; c0 += kDnBatch * LPR) {
+            if (c0 != sub) down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o0, C, c0, w);
+#pragma unroll
+            for (int b = 0; b < kDnBatch; ++b) {
+                const int c = c0 + b * LPR;
+                if (c >= C) break;
+#pragma unroll
+                for (int q = 0; q < kPairsDN; ++q) {
+                    if (!pvalid[q]) continue;
+                    XChunk<F, LO> x;
+                    load_x<F, LO>(act, n, pslot[q] * C + c, x);
+                    acc[q] += dot_chunk<F, LO>(w[b][q], x);
+                }
+            }
+        }
+        done(0, acc);
+        return;
+    }
+    const int nc = (C + kDnBatch * LPR - 1) / (kDnBatch * LPR);   // batches per block
+    float acc[kPairsDN];
+#pragma unroll
+    for (int q = 0; q < kPairsDN; ++q) acc[q] = 0.0f;
+    int blk = 0, ci = 0;
+    for (int it = nb * nc; it > 0; --it) {
+        Pre nxt[kDnBatch][kPairsDN];
+        const bool last = ci + 1 == nc;                   // of this block (uniform)
+        if (it > 1)
+            down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o0 + (last ? blk + 1 : blk) * rstep, C,
+                               sub + (last ? 0 : (ci + 1) * kDnBatch * LPR), nxt);
 #pragma unroll
         for (int b = 0; b < kDnBatch; ++b) {
-            const int c = c0 + b * LPR;
+            const int c = sub + (ci * kDnBatch + b) * LPR;
             if (c >= C) break;
 #pragma unroll
             for (int q = 0; q < kPairsDN; ++q) {
@@ -694,6 +786,21 @@ __device__ __forceinline__ void down_rows(const DecodeArgs& a, const int* pslot,
                 load_x<F, LO>(act, n, pslot[q] * C + c, x);
                 acc[q] += dot_chunk<F, LO>(w[b][q], x);
             }
+        }
+        if (last) {
+            done(blk, acc);
+#pragma unroll
+            for (int q = 0; q < kPairsDN; ++q) acc[q] = 0.0f;
+            ++blk;
+            ci = 0;
+        } else {
+            ++ci;
+        }
+        if (it > 1) {
+#pragma unroll
+            for (int b = 0; b < kDnBatch; ++b)
+#pragma unroll
+                for (int q = 0; q < kPairsDN; ++q) w[b][q] = nxt[b][q];
         }
     }
 }
@@ -708,14 +815,15 @@ __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* 
     const int KS = K + (SH ? 1 : 0);
     const int C = I / Chunk<F>::CH;
     const int RB = a.dn_rb;
-    const int nb = (H + RB - 1) / RB;
-    const int t = j / nb;
-    const int o_base = (j % nb) * RB;
+    const int blocks = (H + RB - 1) / RB, groups = (blocks + a.dn_nb - 1) / a.dn_nb;   // of dn_nb row blocks
+    const int t = j / groups;
+    const int o_base = j % groups * a.dn_nb * RB;
+    const int nb = min(a.dn_nb, blocks - j % groups * a.dn_nb);
     const int grp = threadIdx.x / LPR;
     const int sub = threadIdx.x % LPR;
     const int npairs = KS * RB;
     const int n = KS * I;
-    float* part = reinterpret_cast<float*>(lds + act_words<F>(n));   // [KS][RB]
+    float* part = reinterpret_cast<float*>(lds + act_words<F>(n));   // [nb][KS][RB]
     __shared__ float slot_w[32];   // routed weight per slot, 0 = skipped
     __shared__ int slot_e[32];     // expert per slot, -1 = skipped
     GRIM_TS(a, 2, 0);
@@ -737,54 +845,53 @@ __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* 
     __syncthreads();
     GRIM_TS(a, 2, 1);
     int pslot[NP], prow[NP];
-    int64_t wrow[NP];
+    int64_t wbase[NP];
     bool pshared[NP], pvalid[NP];
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
         const int p = grp + q * G;
         pslot[q] = p % KS;
         prow[q] = p / KS;
-        const int o = min(o_base + prow[q], H - 1);
-        pvalid[q] = p < npairs && o_base + prow[q] < H;
+        pvalid[q] = p < npairs;
         pshared[q] = SH && pslot[q] >= K;
-        wrow[q] = o;
+        wbase[q] = 0;
         if (pvalid[q] && !pshared[q]) {
             const int e = slot_e[pslot[q]];
             if (e < 0) pvalid[q] = false;
-            else wrow[q] = int64_t(e) * H + o;
+            else wbase[q] = int64_t(e) * H;
         }
     }
-    float acc[NP];
     Pre w[kDnBatch][NP];
-#pragma unroll
-    for (int q = 0; q < NP; ++q) acc[q] = 0.0f;
     // (2) the first batch of weights, then h into LDS while they fly
-    down_issue<F, LPR>(a, pvalid, pshared, wrow, C, sub, w);
+    down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o_base, C, sub, w);
     float gate_sh = 1.0f;
-    if (SH && a.gate_in && int(threadIdx.x) < RB) gate_sh = a.gate_in[t];
+    if (SH && a.gate_in) gate_sh = a.gate_in[t];
     const bool lo_pass = a.fmt_h ? h_store<F>(hr, hsrc, n, lds)
                                   : stage_act<F, 4>(a.h + int64_t(t) * n, n, lds);
     GRIM_TS(a, 2, 2);
-    if (lo_pass) down_rows<F, LPR, true>(a, pslot, pvalid, pshared, wrow, C, sub, lds, n, w, acc);
-    else down_rows<F, LPR, false>(a, pslot, pvalid, pshared, wrow, C, sub, lds, n, w, acc);
+    auto done = [&](int blk, const float (&acc)[NP]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < NP; ++q) {
-        const float v = group_sum<LPR>(acc[q]);
-        const int p = grp + q * G;
-        if (sub == 0 && p < npairs) part[pslot[q] * RB + prow[q]] = pvalid[q] ? v : 0.0f;
-    }
+        for (int q = 0; q < NP; ++q) {
+            const float v = group_sum<LPR>(acc[q]);
+            const int p = grp + q * G;
+            if (sub == 0 && p < npairs) part[(blk * KS + pslot[q]) * RB + prow[q]] = pvalid[q] ? v : 0.0f;
+        }
+    };
+    if (lo_pass) down_rows<F, LPR, true>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
+    else down_rows<F, LPR, false>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
     GRIM_TS(a, 2, 3);
     __syncthreads();
-    for (int r = threadIdx.x; r < RB; r += blockDim.x) {
+    for (int r = threadIdx.x; r < nb * RB; r += blockDim.x) {
         const int o = o_base + r;
         if (o >= H) continue;
+        const float* pr = part + (r / RB * KS) * RB + r % RB;
         float total = 0.0f;
         for (int s = 0; s < K; ++s) {
             const float rw = slot_w[s];
             if (rw == 0.0f) continue;
-            total = __builtin_fmaf(rw, part[s * RB + r], total);
+            total = __builtin_fmaf(rw, pr[s * RB], total);
         }
-        if (SH) total = __builtin_fmaf(gate_sh, part[K * RB + r], total);
+        if (SH) total = __builtin_fmaf(gate_sh, pr[K * RB], total);
         a.y[int64_t(t) * H + o] = total;
     }
     GRIM_TS(a, 2, 4);
