@@ -70,6 +70,107 @@ __device__ __forceinline__ uint32_t load_s2(const uint8_t* p) {
     return uint32_t(*reinterpret_cast<const uint16_t*>(p));
 }
 
+// fp32 values staged in LDS for load_x32's consumers: value 32 c + 4 q + i
+// at float4 index q (C + 1) + c, so that the lanes of a row (consecutive
+// chunks c) read 16 bytes each without bank conflicts, and so do the writes.
+// Read straight from memory, a lane's 32 consecutive values are eight loads
+// of 64 lines each: eight times what the row's weights cost the address unit.
+__device__ __forceinline__ void stage_x32(const float* __restrict__ src, int n, float4* dst) {
+    const int C = n / 32;
+    for (int f = threadIdx.x; f < n / 4; f += blockDim.x)
+        dst[(f & 7) * (C + 1) + (f >> 3)] = reinterpret_cast<const float4*>(src)[f];
+}
+__device__ __forceinline__ void load_x32_lds(const float4* s, int C, int c, float* x) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const float4 v = s[q * (C + 1) + c];
+        x[4 * q] = v.x; x[4 * q + 1] = v.y; x[4 * q + 2] = v.z; x[4 * q + 3] = v.w;
+    }
+}
+__host__ __device__ constexpr int stage_floats(int n) { return (n / 32 + 1) * 32; }   // LDS floats of n staged values
+
+// gate + up, x staged in LDS: a work-group takes nb row blocks of one (token,
+// slot), so its expert and block are uniform; per block each lane group owns
+// 2 (gate row, up row) pairs, the blocks' chunks one stream with the next
+// chunk in flight.  The sums are those of tmoe_gate_up_kernel.  Measured
+// (kernel, H 2048, I 768, top-8 of 128): 2 tokens 14.9 -> 11.7 us, 1 token
+// 8.7 -> 7.6; 8 tokens, H 4096, I 1536, top-10: 168 -> 115.
+template <int LPR>
+__global__ __launch_bounds__(kTmThreads) void tmoe_gate_up_staged(TmoeArgs a, int nb) {
+    constexpr int kGroups = kWave / LPR, kPairs = 2;
+    constexpr int kPerBlock = (kTmThreads / kWave) * kGroups * kPairs;   // divides I (a multiple of 128)
+    extern __shared__ __attribute__((aligned(16))) float4 xs[];
+    const int H = a.H, I = a.I, K = a.K, C = H / 32;
+    const int blocks = I / kPerBlock, groups = (blocks + nb - 1) / nb;
+    const int t = blockIdx.x / (K * groups), slot = blockIdx.x / groups % K, b0 = blockIdx.x % groups * nb;
+    const int n = min(nb, blocks - b0);
+    const int lane = threadIdx.x & (kWave - 1), sub = lane % LPR;
+    const int row0 = b0 * kPerBlock + ((threadIdx.x / kWave) * kGroups + lane / LPR) * kPairs;
+    const int e = a.expert[int64_t(t) * K + slot];
+    const bool on = e >= 0 && e < a.E;   // uniform
+    float* ht = a.h + int64_t(t) * K * I + int64_t(slot) * I;
+    if (!on) {
+        for (int i = threadIdx.x; i < n * kPerBlock; i += kTmThreads) ht[b0 * kPerBlock + i] = 0.0f;
+        return;
+    }
+    const uint8_t* blk = a.eptr[e];
+    const float sgf = reinterpret_cast<const float*>(blk + a.gsc)[0];
+    const float suf = reinterpret_cast<const float*>(blk + a.gsc)[1];
+    const uint8_t* wp = blk + a.gu_p + int64_t(row0) * (H / 2);
+    const uint8_t* sp = blk + a.gu_s + int64_t(row0) * (H / 16);
+    const int64_t up_p = int64_t(I) * (H / 2), up_s = int64_t(I) * (H / 16);
+    struct Pre {
+        uint4 g[kPairs], u[kPairs];
+        uint32_t sg[kPairs], su[kPairs];
+    };
+    auto load = [&](Pre& p, int b, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < kPairs; ++r) {
+            const uint8_t* w = wp + int64_t(b * kPerBlock + r) * (H / 2) + c * 16;
+            const uint8_t* s = sp + int64_t(b * kPerBlock + r) * (H / 16) + c * 2;
+            p.g[r] = *reinterpret_cast<const uint4*>(w);
+            p.u[r] = *reinterpret_cast<const uint4*>(w + up_p);
+            p.sg[r] = load_s2(s);
+            p.su[r] = load_s2(s + up_s);
+        }
+    };
+    Pre cur, nxt;
+    load(cur, 0, sub < C ? sub : C - 1);
+    stage_x32(a.x + int64_t(t) * H, H, xs);
+    __syncthreads();
+    float ga[kPairs] = {}, ua[kPairs] = {};
+    const int nc = (C + LPR - 1) / LPR;
+    int b = 0, ci = 0;
+    for (int it = n * nc; it > 0; --it) {
+        const bool last = ci + 1 == nc;   // of this block (uniform)
+        const int c = sub + ci * LPR, cn = sub + (last ? 0 : (ci + 1) * LPR);
+        if (it > 1) load(nxt, last ? b + 1 : b, cn < C ? cn : C - 1);
+        if (c < C) {
+            float x[32];
+            load_x32_lds(xs, C, c, x);
+#pragma unroll
+            for (int r = 0; r < kPairs; ++r) {
+                ga[r] += nv_dot32(cur.g[r], cur.sg[r], x);
+                ua[r] += nv_dot32(cur.u[r], cur.su[r], x);
+            }
+        }
+        if (last) {
+#pragma unroll
+            for (int r = 0; r < kPairs; ++r) {
+                const float g = group_sum<LPR>(ga[r]);
+                const float u = group_sum<LPR>(ua[r]);
+                if (sub == 0) ht[row0 + b * kPerBlock + r] = silu(g * sgf) * (u * suf);
+                ga[r] = ua[r] = 0.0f;
+            }
+            ++b;
+            ci = 0;
+        } else {
+            ++ci;
+        }
+        if (it > 1) cur = nxt;
+    }
+}
+
 // gate + up: each lane group owns 2 (gate row, up row) pairs of one
 // (token, slot); h[t][slot*I + i] = silu(g * s_gate) * (u * s_up), 0 for a
 // slot routed to no expert of this table (id < 0 or >= E).
@@ -248,6 +349,121 @@ __global__ __launch_bounds__(kTmThreads) void tmoe_down_kernel(TmoeArgs a) {
     }
 }
 
+// The same with h staged in LDS and nb blocks of output rows per work-group,
+// each block's weights requested before the previous one's are multiplied
+// (top_k <= 16).  LDS: h of every slot, then the dots [K][nb kPerBlock].
+// Measured (kernel): 5 tokens, H 2688, I 768, top-6: 33.5 -> 21.6 us; 8
+// tokens, H 4096, I 1536, top-10: 294 -> 167; 1 token, H 2048: 8.7 either way.
+// NW waves of KW slots: more than 8 slots take 8 waves, not four slots a wave
+// (308 registers).
+template <int LPR, int KW, int NW>
+__global__ __launch_bounds__(NW * kWave) void tmoe_down_staged(TmoeArgs a, int nb) {
+    constexpr int kWaves = NW, kGroups = kWave / LPR, kRows = 2, kPerBlock = kGroups * kRows;
+    extern __shared__ __attribute__((aligned(16))) float4 hs[];
+    const int H = a.H, I = a.I, K = a.K, C = I / 32, HF = stage_floats(I) / 4;   // float4s per slot
+    float* part = reinterpret_cast<float*>(hs + K * HF);
+    const int blocks = (H + kPerBlock - 1) / kPerBlock, groups = (blocks + nb - 1) / nb;
+    const int t = blockIdx.x / groups, b0 = blockIdx.x % groups * nb;
+    const int n = min(nb, blocks - b0), PR = nb * kPerBlock;   // rows of part
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), sub = lane % LPR, g = lane / LPR;
+    const int o0 = b0 * kPerBlock + g * kRows;
+    __shared__ float coef[kTmMaxK];       // w_s * s_down
+    __shared__ int on_slot[kTmMaxK];      // 0: slot skipped
+    int ev[KW];
+    float rv[KW], sdv[KW];
+    const uint8_t* bv[KW];
+    bool onv[KW];
+#pragma unroll
+    for (int j = 0; j < KW; ++j) {
+        const int s = wave + j * kWaves;
+        const int64_t sc = int64_t(t) * K + (s < K ? s : K - 1);
+        ev[j] = a.expert[sc];
+        rv[j] = a.weight[sc];
+    }
+    for (int s = 0; s < K; ++s) stage_x32(a.h + (int64_t(t) * K + s) * I, I, hs + s * HF);
+#pragma unroll
+    for (int j = 0; j < KW; ++j) {
+        const int s = wave + j * kWaves;
+        onv[j] = s < K && ev[j] >= 0 && ev[j] < a.E && rv[j] != 0.0f;
+        bv[j] = a.eptr[onv[j] ? ev[j] : 0];
+    }
+#pragma unroll
+    for (int j = 0; j < KW; ++j) sdv[j] = reinterpret_cast<const float*>(bv[j] + a.gsc)[2];
+    struct Pre {
+        uint4 p[KW][kRows];
+        uint32_t s[KW][kRows];
+    };
+    // (a skipped slot reads a valid block, masked)
+    auto load = [&](Pre& w, int b, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < KW; ++j)
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) {
+                const int o = min(o0 + b * kPerBlock + r, H - 1);
+                w.p[j][r] = *reinterpret_cast<const uint4*>(bv[j] + a.dn_p + int64_t(o) * (I / 2) + c * 16);
+                w.s[j][r] = load_s2(bv[j] + a.dn_s + int64_t(o) * (I / 16) + c * 2);
+            }
+    };
+    Pre cur, nxt;
+    load(cur, 0, sub < C ? sub : C - 1);
+#pragma unroll
+    for (int j = 0; j < KW; ++j) {
+        const int s = wave + j * kWaves;
+        if (s < K && lane == 0) {
+            coef[s] = onv[j] ? rv[j] * sdv[j] : 0.0f;
+            on_slot[s] = onv[j] ? 1 : 0;
+        }
+    }
+    __syncthreads();
+    float acc[KW][kRows] = {};
+    const int nc = (C + LPR - 1) / LPR;
+    int b = 0, ci = 0;
+    for (int it = n * nc; it > 0; --it) {
+        const bool last = ci + 1 == nc;   // of this block (uniform)
+        const int c = sub + ci * LPR, cn = sub + (last ? 0 : (ci + 1) * LPR);
+        if (it > 1) load(nxt, last ? b + 1 : b, cn < C ? cn : C - 1);
+        if (c < C) {
+#pragma unroll
+            for (int j = 0; j < KW; ++j) {
+                const int s = wave + j * kWaves;
+                float x[32];
+                load_x32_lds(hs + (s < K ? s : K - 1) * HF, C, c, x);
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) {
+                    const float d = nv_dot32(cur.p[j][r], cur.s[j][r], x);
+                    acc[j][r] += onv[j] ? d : 0.0f;
+                }
+            }
+        }
+        if (last) {
+#pragma unroll
+            for (int j = 0; j < KW; ++j) {
+                const int s = wave + j * kWaves;
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) {
+                    const float d = group_sum<LPR>(acc[j][r]);
+                    if (onv[j] && sub == 0) part[s * PR + b * kPerBlock + g * kRows + r] = d;
+                    acc[j][r] = 0.0f;
+                }
+            }
+            ++b;
+            ci = 0;
+        } else {
+            ++ci;
+        }
+        if (it > 1) cur = nxt;
+    }
+    __syncthreads();
+    for (int row = threadIdx.x; row < n * kPerBlock; row += NW * kWave) {
+        const int o = b0 * kPerBlock + row;
+        if (o >= H) continue;
+        float total = 0.0f;
+        for (int s = 0; s < K; ++s)
+            if (on_slot[s]) total = __builtin_fmaf(coef[s], part[s * PR + row], total);
+        a.y[int64_t(t) * H + o] = total;
+    }
+}
+
 // Prefill on one expert block: the block's NVFP4 rows decoded into bf16
 // scratch rows (exact: an e2m1 value times an E4M3 scale has at most 6
 // significant bits), which the grouped bf16 GEMM then reads; the fp32
@@ -363,9 +579,39 @@ static int lanes_for(int chunks) {
         default: GRIM_TM_LAUNCH(KERNEL, 64, GRID); break;                                          \
     }
 
+// Row blocks per work-group of the staged kernels: as many as leave at least
+// two work-groups per CU.
+constexpr int kTmItems = 512, kTmMaxNB = 16;
+static int tm_nb(int64_t units, int blocks) {
+    int nb = 1;
+    while (nb < kTmMaxNB && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= kTmItems) nb *= 2;
+    return nb;
+}
+// The staged kernels' LDS limit, two work-groups per CU (the activations in
+// fp32; larger ones are read from memory by the others).
+constexpr size_t kTmStageMax = 80 * 1024;
+
 hipError_t tmoe_gate_up(hipStream_t st, const TmoeArgs& a) {
     if (a.M <= 0) return hipSuccess;
     const int lpr = lanes_for(a.H / 32);
+    const size_t lds = size_t(stage_floats(a.H)) * 4;
+    if (lds <= kTmStageMax) {
+        const int blocks = a.I / ((kTmThreads / kWave) * (kWave / lpr) * 2);
+        const int nb = tm_nb(int64_t(a.M) * a.K, blocks);
+        const dim3 grid(unsigned(int64_t(a.M) * a.K * ((blocks + nb - 1) / nb)));
+#define GRIM_TMG_STAGED(L) \
+    case L: hipLaunchKernelGGL((tmoe_gate_up_staged<L>), grid, dim3(kTmThreads), lds, st, a, nb); break
+        switch (lpr) {   // H % 128 == 0: at least four chunks a row
+            GRIM_TMG_STAGED(4);
+            GRIM_TMG_STAGED(8);
+            GRIM_TMG_STAGED(16);
+            GRIM_TMG_STAGED(32);
+            GRIM_TMG_STAGED(64);
+            default: return hipErrorInvalidValue;
+        }
+#undef GRIM_TMG_STAGED
+        return hipGetLastError();
+    }
     const int per_block = (kTmThreads / kWave) * (kWave / lpr) * 2;
     const dim3 grid(unsigned(int64_t(a.M) * ((a.K * a.I + per_block - 1) / per_block)));
     GRIM_TM_SWITCH(tmoe_gate_up_kernel, lpr, grid);
@@ -390,6 +636,32 @@ hipError_t tmoe_down(hipStream_t st, const TmoeArgs& a) {
     const dim3 grid(unsigned(int64_t(a.M) * ((a.H + per_block - 1) / per_block)));
     const int need = (a.K + kTmThreads / kWave - 1) / (kTmThreads / kWave);
     const int kw = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+    {
+        const int blocks = (a.H + per_block - 1) / per_block, nb = tm_nb(a.M, blocks);
+        const size_t lds = size_t(a.K) * (stage_floats(a.I) + nb * per_block) * 4;
+        if (a.K <= 16 && lds <= kTmStageMax) {
+            const dim3 sgrid(unsigned(int64_t(a.M) * ((blocks + nb - 1) / nb)));
+#define GRIM_TMD_GO(L, KW, NW) \
+    hipLaunchKernelGGL((tmoe_down_staged<L, KW, NW>), sgrid, dim3(NW * kWave), lds, st, a, nb)
+#define GRIM_TMD_STAGED(L)              \
+    case L:                             \
+        if (a.K <= 4) GRIM_TMD_GO(L, 1, 4);      \
+        else if (a.K <= 8) GRIM_TMD_GO(L, 2, 4); \
+        else GRIM_TMD_GO(L, 2, 8);      \
+        break
+            switch (lpr) {   // I % 128 == 0: at least four chunks a row
+                GRIM_TMD_STAGED(4);
+                GRIM_TMD_STAGED(8);
+                GRIM_TMD_STAGED(16);
+                GRIM_TMD_STAGED(32);
+                GRIM_TMD_STAGED(64);
+                default: return hipErrorInvalidValue;
+            }
+#undef GRIM_TMD_STAGED
+#undef GRIM_TMD_GO
+            return hipGetLastError();
+        }
+    }
     switch (lpr) {
         case 1: GRIM_TMD_KW(1); break;
         case 2: GRIM_TMD_KW(2); break;
