@@ -15,8 +15,9 @@
 //     64-byte piece (a "segment": 128 K of 4-bit codes, 32 K of bf16) and
 //     each 16-byte register holds the operands of J MFMA steps (4 for
 //     4-bit, 1 for bf16).  A stage is SP segments of the wave's rows, double
-//     buffered in registers (SP 2 against 4 on MXFP4, K 2048, 8 rows per
-//     expert: 126 -> 116 us; SP 1: 156 us).
+//     buffered in registers (MXFP4 down, 128 experts x 8 rows, K 2048, N 4096:
+//     SP 2 116 us, SP 4 132: more lines in flight than the L2 holds; SP 1 a
+//     third slower).
 //   - Activations (bf16 rows, one or two planes) come through LDS by
 //     buffer_load ... lds, double buffered, gathered by row through the
 //     route -> token map; 16-byte slots XOR-swizzled by row so that the
@@ -32,13 +33,12 @@
 // one operation fewer, would lose three more bits to the offset.)
 //
 // Measured (one MI355X, kernel alone): MXFP4, 128 experts x 8 rows, K = N =
-// 2880: gate_up 285 us = 3.96 TB/s of weights, down 155 us; the same with
-// loads only 264 / 134 us: rows of 1440 bytes put odd rows' pieces across
-// memory lines (K 2048: 116 us = 4.9 TB/s, loads only 109).  bf16, 64 experts
-// x 9 rows, K 2048: gate_up 110 us = 4.9 TB/s, down 47 us = 5.7 TB/s.  INT4,
-// 64 experts x 1 row, K 2048: gate_up 28 us = 5.0 TB/s.  32 experts x 512
-// rows, K = N = 2880 MXFP4: gate_up 680 us = 0.80 PFLOP/s, down (two planes)
-// 625 us = 0.87.  The 128-row tile kernel (gemm.hip) before it, 1000 tokens
+// 2880: gate_up 259 us = 4.4 TB/s of weights, down 143 us (rows of 1440 bytes
+// put odd rows' pieces across memory lines); K 4096, N 2048: gate_up 228 us =
+// 5.0 TB/s.  bf16, 64 experts x 9 rows, K 2048: gate_up 112 us = 4.8 TB/s,
+// down 46 us = 5.8 TB/s.  INT4, 128 experts x 1 row, K 4096, N 1024: gate_up
+// 97 us = 5.7 TB/s.  32 experts x 512 rows, K = N = 2880 MXFP4: gate_up 680
+// us = 0.80 PFLOP/s, down (two planes) 625 us = 0.87.  The 128-row tile kernel (gemm.hip) before it, 1000 tokens
 // of the layer with Zipf(1.1) popularity: gate_up 676 -> 375 us, down 596 ->
 // 257 us.
 #include "gemm_wreg.hpp"
@@ -245,14 +245,18 @@ __device__ __forceinline__ void wreg_tile(const WregArgs& a, const WregItem& it,
     // stage st's weights (K past the row's end reads as zero), and its
     // chunk of scales when that is not the one at hand
     auto load_w = [&](Stage& S, int st) __attribute__((always_inline)) {
+        // (row blocks outermost: the segments of a row one after the other, so
+        // that the pieces of a memory line are requested together: MXFP4, 128
+        // experts x 8 rows, K = N = 2880: 286 -> 259 us; K 4096, N 2048: 245
+        // -> 228)
 #pragma unroll
-        for (int s = 0; s < SP; ++s) {
-            const int seg = st * SP + s;
-            const bool in = seg * SEGK + g * (SEGK / 4) < K;
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
+            for (int s = 0; s < SP; ++s) {
+                const int seg = st * SP + s;
+                const bool in = seg * SEGK + g * (SEGK / 4) < K;
                 S.b[s][rb] = __builtin_amdgcn_raw_buffer_load_b128(rW, in ? woff[rb] : kWregNoLoad, seg * 64, 0);
-        }
+            }
         if constexpr (CW != 0) {
             const int ch = st * SP / 16;
             if (st < nstg && ch != chunk_n) {   // uniform
