@@ -611,12 +611,17 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
                         size_t workspace_bytes, int roles, int shard_begin = 0, int shard_count = 0);
 
 // The plan of a call whose workspace holds `bytes`: the register-weight
-// products where the call takes them and their buffers fit (a caller of
-// forward_noalloc has a fixed size), else the slot or grouped kernels.
+// products where the call takes them and their buffers fit, else the slot or
+// grouped kernels.  The others' buffers have to fit as well (the token rows
+// gathered in place make these the smaller ones for MXFP4 and bf16): whether
+// a workspace is large enough does not depend on the products that run.
 static PlanKind plan_kind(const grim_moe_layer* L, int tokens, int regime, size_t bytes) {
     Plan p{};
-    if (use_wreg(L, tokens, regime) && carve(L, tokens, PlanKind::kWreg, nullptr, p) <= bytes) return PlanKind::kWreg;
-    return use_gemv(L, tokens, regime) ? PlanKind::kSlots : PlanKind::kGrouped;
+    const PlanKind other = use_gemv(L, tokens, regime) ? PlanKind::kSlots : PlanKind::kGrouped;
+    return use_wreg(L, tokens, regime) && carve(L, tokens, other, nullptr, p) <= bytes &&
+                   carve(L, tokens, PlanKind::kWreg, nullptr, p) <= bytes
+               ? PlanKind::kWreg
+               : other;
 }
 
 extern "C" int grimoire_moe_forward(void* stream, const grim_moe_layer* L,
