@@ -171,7 +171,7 @@ bool wreg_ok(const grim_moe_layer* L, int T) {
 
 // ... and the call takes them: MXFP4 and bf16 experts wherever the grouped
 // GEMM would run (1000 tokens of 128 MXFP4 experts, H = I = 2880: 1300 ->
-// 660 us a layer; 150 tokens of 64 bf16 experts: 299 -> 225 us).  INT4
+// 593 us a layer; 150 tokens of 64 bf16 experts: 299 -> 188 us).  INT4
 // experts, up to the two routes per expert that INT4 batches are taken for:
 // above 64 routes always (the vector-ALU grouped GEMV otherwise: 20 tokens x
 // top-8 of 128, H 2048, I 768: 304 -> 76 us), below when the bytes that the

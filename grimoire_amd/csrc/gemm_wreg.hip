@@ -38,9 +38,9 @@
 // 5.0 TB/s.  bf16, 64 experts x 9 rows, K 2048: gate_up 112 us = 4.8 TB/s,
 // down 46 us = 5.8 TB/s.  INT4, 128 experts x 1 row, K 4096, N 1024: gate_up
 // 97 us = 5.7 TB/s.  32 experts x 512 rows, K = N = 2880 MXFP4: gate_up 680
-// us = 0.80 PFLOP/s, down (two planes) 625 us = 0.87.  The 128-row tile kernel (gemm.hip) before it, 1000 tokens
-// of the layer with Zipf(1.1) popularity: gate_up 676 -> 375 us, down 596 ->
-// 257 us.
+// us = 0.80 PFLOP/s, down (two planes) 625 us = 0.87.  1000 tokens of the
+// layer (128 experts, top-4, K = N = 2880, Zipf(1.1) popularity): gate_up 676
+// -> 341 us, down 596 -> 232 us against the 128-row tile kernel (gemm.hip).
 #include "gemm_wreg.hpp"
 
 #include "dispatch_one.hpp"

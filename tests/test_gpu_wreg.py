@@ -77,3 +77,53 @@ def test_mxfp4_scale_windows(gpu, H, I):
 def test_int4(gpu, H, I, zeros, fp32_x):
     print(f"wreg int4 H={H} I={I} zeros={zeros} fp32_x={fp32_x}", flush=True)
     _run(gpu, configs.Config("t", 35, H, 36, 2, I, "int4", shared=True), seed=H, zeros=zeros, fp32_x=fp32_x)
+
+
+@pytest.mark.parametrize("fmt,T,regime", [("int4", 35, 0), ("bf16", 150, 2), ("mxfp4", 1500, 2)])
+def test_shards_sum_to_the_layer(gpu, fmt, T, regime):
+    """Shards of 12 of 36 experts (routes elsewhere are -1), both dispatch
+    routes: each y is the layer's part, the sum the whole layer."""
+    print(f"wreg shards {fmt} T={T}", flush=True)
+    cfg = configs.Config("t", T, 512, 36, 6 if T > 1000 else 2, 640, fmt)
+    Lg = configs.make_workload(cfg, "cpu", seed=T).layer.to(gpu)
+    x = configs.make_x(cfg, "cpu", seed=T).to(gpu)
+    rp = configs.route_params(cfg, None)
+    y = torch.empty(T, cfg.H, device=gpu)
+    ops.MoeForward(Lg, T, rp, regime)(x, y)
+    total = torch.zeros(T, cfg.H, dtype=torch.float64, device=gpu)
+    for b in (0, 12, 24):
+        ys = torch.full((T, cfg.H), float("nan"), device=gpu)
+        ops.MoeForward(Lg.shard(b, 12, shared=False), T, rp, regime).shard(x, ys, b, 12)
+        total += ys.double()
+    torch.cuda.synchronize()
+    assert torch.isfinite(total).all()
+    assert rel_l2(total.float().cpu(), y.cpu()) <= TOL
+
+
+@pytest.mark.parametrize("fmt,T,regime", [("int4", 16, 0), ("int4", 35, 0), ("bf16", 150, 2), ("mxfp4", 1500, 2)])
+def test_graph_replays(gpu, fmt, T, regime):
+    """Captured once, replayed on new inputs between eager calls: the bits of
+    the eager call."""
+    print(f"wreg graph {fmt} T={T}", flush=True)
+    # T = 16: the rule on bytes (55 MB of slot reads), top-k in the dispatch launch
+    cfg = configs.Config("t", T, 2048 if T == 16 else 512, 36, 6 if T > 1000 else 2, 640, fmt, shared=T != 16)
+    Lg = configs.make_workload(cfg, "cpu", seed=T).layer.to(gpu)
+    fwd = ops.MoeForward(Lg, T, configs.route_params(cfg, None), regime)
+    xs = [configs.make_x(cfg, "cpu", seed=s).to(gpu) for s in (1, 2)]
+    x, y, ye = xs[0].clone(), torch.empty(T, cfg.H, device=gpu), torch.empty(T, cfg.H, device=gpu)
+    fwd(x, y)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        fwd(x, y, stream=s)
+    for rep in range(3):
+        for xi in xs:
+            fwd(xi, ye)
+            x.copy_(xi)
+            y.fill_(float("nan"))
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, ye), f"replay {rep}"
