@@ -17,6 +17,7 @@ Source kinds (one checkpoint projection [out][in] each):
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from dataclasses import dataclass
 from typing import Optional, Sequence, Tuple
 
@@ -87,6 +88,19 @@ def stacked(fmt: int, N: int, K: int, group: int, device) -> Weight:
     raise ValueError(f"no ingestion into format {fmt}")
 
 
+def _table(srcs: Sequence[Projection]) -> C.Array:
+    """The projections' structs as one array, packed in one call: a ctypes
+    object per projection was a third of a layer's ingestion (384 projections,
+    2048 x 768: 379 -> 250 us)."""
+    v = []
+    for p in srcs:
+        w, z, s = p.weight, p.zeros, p.scales
+        v += (p.kind, p.in_, p.out, p.group, 0 if w is None else w.data_ptr(),
+              0 if z is None else z.data_ptr(), 0 if s is None else s.data_ptr())
+    n = len(srcs)
+    return (_abi.ExpertSrc * n).from_buffer_copy(struct.pack("4i3Q" * n, *v))
+
+
 def ingest_projection(src: Projection, dst: Weight, row0: int, stream=None) -> None:
     s, d = src.struct(), dst.struct()
     check(lib().grimoire_moe_ingest_projection(_stream(stream), C.byref(s), C.byref(d), row0),
@@ -98,7 +112,7 @@ def ingest_projections(srcs: Sequence[Projection], dst: Weight, row0: Sequence[i
     """Projections of one kind and shape into one stacked weight, batched
     (GPTQ: 64 per launch)."""
     n = len(srcs)
-    arr = (_abi.ExpertSrc * n)(*[p.struct() for p in srcs])
+    arr = _table(srcs)
     rows = (C.c_int32 * n)(*row0)
     d = dst.struct()
     check(lib().grimoire_moe_ingest_projections(_stream(stream), arr, C.cast(rows, C.c_void_p), n,
