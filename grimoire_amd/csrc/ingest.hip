@@ -29,17 +29,42 @@ namespace grim {
 constexpr int kTile = 64;        // words per tile side
 constexpr int kIngThreads = 256;
 
-// Projection z of the batch: out32[o * out_stride + r] = in32[r * C + o]
-// for r < R, o < C, out32 = the payload rows from row0[z].
-__global__ __launch_bounds__(kIngThreads) void transpose_u32(const IngestGptq a) {
+// Scales and zero points of projection z, one thread per (group g, output
+// o), o fastest: reads of the checkpoint rows are coalesced; the
+// [out][groups] writes are short rows.
+__device__ __forceinline__ void gptq_meta(const IngestGptq& a, int z, int64_t i) {
+    const int out = a.out, groups = a.in / a.group;
+    if (i >= int64_t(out) * groups) return;
+    const int g = int(i / out), o = int(i % out);
+    const uint16_t s = a.scales[z][int64_t(g) * out + o];
+    const uint32_t zw = a.qzeros[z][int64_t(g) * (out >> 3) + (o >> 3)];
+    const int64_t d = int64_t(a.row0[z] + o) * a.dst_rs + g;
+    a.dst_scales[d] = a.keep_f16 ? s : f32_to_bf16(f16_to_f32(s));
+    a.dst_zeros[d] = uint8_t(((zw >> ((o & 7) * 4)) & 0xFu) + 1u);
+}
+
+// Projection z = blockIdx.y of the batch.  The first meta_blocks work-groups
+// of a projection do its scales and zero points, the others one transpose
+// tile each: out32[o * out_stride + r] = in32[r * C + o] for r < R, o < C,
+// out32 = the payload rows from row0[z].  In a launch of their own the
+// scales were bound by the latency of their short writes (64 projections of
+// 768 x 2048: 7.6 us after the transposes' 23); here they run beside them
+// (128 projections 47.5 us = 4.4 TB/s read + written; a layer of 384 in
+// three launches instead of twelve, 250 -> 217 us with the host's part).
+__global__ __launch_bounds__(kIngThreads) void gptq_ingest(const IngestGptq a, int meta_blocks, int col_tiles) {
     __shared__ uint32_t tile[kTile][kTile + 1];
-    const int z = blockIdx.z;
+    const int z = blockIdx.y;
+    if (int(blockIdx.x) < meta_blocks) {
+        gptq_meta(a, z, int64_t(blockIdx.x) * kIngThreads + threadIdx.x);
+        return;
+    }
+    const int t = blockIdx.x - meta_blocks;
     const int R = a.in / 8, C = a.out;
     const uint32_t* __restrict__ in = a.qweight[z];
     uint32_t* __restrict__ out =
         reinterpret_cast<uint32_t*>(a.dst_payload + int64_t(a.row0[z]) * a.dst_row_bytes);
     const int64_t out_stride = a.dst_row_bytes / 4;
-    const int c0 = blockIdx.x * kTile, r0 = blockIdx.y * kTile;
+    const int c0 = t % col_tiles * kTile, r0 = t / col_tiles * kTile;
     const int tx = threadIdx.x & (kTile - 1), ty = threadIdx.x / kTile;   // ty in 0..3
     constexpr int kRows = kTile / (kIngThreads / kTile);   // 16 loads per thread, all in flight
     uint32_t v[kRows];
@@ -56,22 +81,6 @@ __global__ __launch_bounds__(kIngThreads) void transpose_u32(const IngestGptq a)
         const int o = c0 + ty + i, r = r0 + tx;
         if (o < C && r < R) out[int64_t(o) * out_stride + r] = tile[tx][ty + i];
     }
-}
-
-// One thread per (group g, output o) of projection blockIdx.y, o fastest:
-// reads of the checkpoint rows are coalesced; the [out][groups] writes are
-// short rows.
-__global__ __launch_bounds__(kIngThreads) void gptq_meta(const IngestGptq a) {
-    const int z = blockIdx.y;
-    const int out = a.out, groups = a.in / a.group;
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= int64_t(out) * groups) return;
-    const int g = int(i / out), o = int(i % out);
-    const uint16_t s = a.scales[z][int64_t(g) * out + o];
-    const uint32_t zw = a.qzeros[z][int64_t(g) * (out >> 3) + (o >> 3)];
-    const int64_t d = int64_t(a.row0[z] + o) * a.dst_rs + g;
-    a.dst_scales[d] = a.keep_f16 ? s : f32_to_bf16(f16_to_f32(s));
-    a.dst_zeros[d] = uint8_t(((zw >> ((o & 7) * 4)) & 0xFu) + 1u);
 }
 
 // compressed-tensors INT4 zero points, or the symmetric 8 when zp == NULL.
@@ -141,12 +150,12 @@ static unsigned stream_blocks(int64_t bytes) {
 
 hipError_t ingest_gptq(hipStream_t st, const IngestGptq& a) {
     if (a.n <= 0 || a.n > kIngBatch) return hipErrorInvalidValue;
-    const int words_r = a.in / 8;   // qweight rows
-    dim3 g1((a.out + kTile - 1) / kTile, (words_r + kTile - 1) / kTile, a.n);
-    hipLaunchKernelGGL(transpose_u32, g1, dim3(kIngThreads), 0, st, a);
+    const int col_tiles = (a.out + kTile - 1) / kTile, row_tiles = (a.in / 8 + kTile - 1) / kTile;
     const int64_t items = int64_t(a.out) * (a.in / a.group);
-    dim3 g2(unsigned((items + kIngThreads - 1) / kIngThreads), a.n);
-    hipLaunchKernelGGL(gptq_meta, g2, dim3(kIngThreads), 0, st, a);
+    const int64_t meta = (items + kIngThreads - 1) / kIngThreads, tiles = int64_t(col_tiles) * row_tiles;
+    if (meta + tiles > 0x7FFFFFFF) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gptq_ingest, dim3(unsigned(meta + tiles), a.n), dim3(kIngThreads), 0, st, a, int(meta),
+                       col_tiles);
     return hipGetLastError();
 }
 

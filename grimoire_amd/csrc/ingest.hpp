@@ -8,8 +8,9 @@ namespace grim {
 
 // GPTQ triples of up to kIngBatch projections of one shape into rows
 // [row0[i], row0[i] + out) of one stacked INT4 / INT4_F16 weight
-// (src/gptq.cpp:56-83).  The table travels in the kernel arguments.
-constexpr int kIngBatch = 64;
+// (src/gptq.cpp:56-83).  The table travels in the kernel arguments, whose
+// limit is 4 KiB.
+constexpr int kIngBatch = 128;
 
 struct IngestGptq {
     const uint32_t* qweight[kIngBatch];  // [in/8][out]
@@ -24,6 +25,7 @@ struct IngestGptq {
     int dst_rs;               // in / group
     int keep_f16;             // 1: fp16 bits kept (INT4_F16); 0: bf16 (INT4)
 };
+static_assert(sizeof(IngestGptq) + 8 <= 4096, "kernel arguments");
 
 struct SignedRegion {
     uint8_t* payload;

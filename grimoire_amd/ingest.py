@@ -110,7 +110,7 @@ def ingest_projection(src: Projection, dst: Weight, row0: int, stream=None) -> N
 def ingest_projections(srcs: Sequence[Projection], dst: Weight, row0: Sequence[int],
                        stream=None) -> None:
     """Projections of one kind and shape into one stacked weight, batched
-    (GPTQ: 64 per launch)."""
+    (GPTQ: 128 per launch)."""
     n = len(srcs)
     arr = _table(srcs)
     rows = (C.c_int32 * n)(*row0)
