@@ -86,18 +86,34 @@ void decode_plan(int fmt, DecodeArgs& a, int roles) {
     // Row blocks per item of the slot kernels: an item's start (its token's
     // activations, the routes or the whole top-k, the first weights: several
     // dependent round trips) is paid once for all of them, as long as the
-    // items still fill the CUs.  Measured, one block an item / grouped to at
-    // least 512 items (256 items; 1024): 3 tokens x top-10 of 512 INT8
-    // experts, H 2048, I 512, 42.8 / 37 us a layer (48; 38); 12 tokens x top-4
-    // of 64 bf16 ones, I 1024, 121 / 95 (99; 109).
+    // items still fill the CUs.  Measured, one block an item / grouped: 3
+    // tokens x top-10 of 512 INT8 experts, H 2048, I 512, 42.0 / 34.2 us a
+    // layer; 12 tokens x top-4 of 64 bf16 ones, I 1024, 121 / 95.
+    auto grouped = [](int64_t units, int blocks, int64_t items, int most) {
+        int nb = 1;
+        while (nb < most && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= items) nb *= 2;
+        return nb;
+    };
     a.gu_nb = a.dn_nb = 1;
     const int dn_blocks = (a.H + a.dn_rb - 1) / a.dn_rb;
-    if (!a.xf)
-        while (a.gu_nb < kGuMaxNB && int64_t(a.M) * KS * ((a.gu_rb + 2 * a.gu_nb - 1) / (2 * a.gu_nb)) >= kSlotItems)
-            a.gu_nb *= 2;
-    if (!a.dn_wave)
-        while (a.dn_nb < kDnMaxNB && int64_t(a.M) * ((dn_blocks + 2 * a.dn_nb - 1) / (2 * a.dn_nb)) >= kSlotItems)
-            a.dn_nb *= 2;
+    // gate_up: where the items hold the top-k (with few slots the start is
+    // short: 4 tokens x top-2, H 3584, I 896 in 672 items 46.7 us, ungrouped
+    // 42.6), or there are a great many (30 tokens x top-2 + shared of 16 bf16
+    // experts, H 2432, I 1536: 17280 items, 340 / 302 us).  Otherwise the
+    // stream's registers cost what the starts saved (INT8, 25 tokens x top-2 +
+    // shared, H 2432, I 960: 117 / 128; bf16, 43 x top-1, H 2240, I 1728: 175 /
+    // 189).
+    if (!a.xf) {
+        const int64_t units = int64_t(a.M) * KS;
+        if (a.route_topk) a.gu_nb = grouped(units, a.gu_rb, KS <= 3 ? 3 * kSlotItems / 2 : kSlotItems, kGuMaxNB);
+        else if (units * a.gu_rb >= 32 * kSlotItems) a.gu_nb = grouped(units, a.gu_rb, 4 * kSlotItems, kGuMaxNB);
+    }
+    // down: staging h is most of a start, so blocks of many rows (few slots)
+    // gain the least: INT8 (whose one-block kernel has five waves per SIMD)
+    // not at all at 16 rows (55 tokens x top-1, H 2752, I 1728: 169 / 175) and
+    // from twice the items at 8 (12 x top-4, H 1216, I 768, 912 items: 46 / 48)
+    if (!a.dn_wave && !(fmt == GRIM_FMT_INT8 && a.dn_rb >= 16))
+        a.dn_nb = grouped(a.M, dn_blocks, fmt == GRIM_FMT_INT8 && a.dn_rb >= 8 ? 2 * kSlotItems : kSlotItems, kDnMaxNB);
     a.NR = (roles & kRoleRouter) ? a.E : 0;
     a.NG = (roles & kRoleGateUp) ? a.M * KS * ((a.gu_rb + a.gu_nb - 1) / a.gu_nb) : 0;
     a.ND = (roles & kRoleDown) ? a.M * ((dn_blocks + a.dn_nb - 1) / a.dn_nb) : 0;

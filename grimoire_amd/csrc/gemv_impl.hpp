@@ -515,14 +515,12 @@ __device__ __forceinline__ void router_item(const DecodeArgs& a, int b) {
 // gate_up rows of nb row blocks of one (token, slot): RU (gate, up) row pairs
 // per lane group and block, the blocks' chunks one stream with the next
 // chunk in flight while this one is multiplied.  cur holds the first; done
-// takes each block's sums.
-template <int F, int LPR, bool LO, class Done>
+// takes each block's sums.  !MANY: nb is 1.
+template <int F, int LPR, bool LO, bool MANY, class Done>
 __device__ __forceinline__ void gate_up_rows(const WView& v, int64_t gbase, int i0, int rstep, int nb, int I,
                                              int C, int sub, const uint32_t* act, int n,
                                              Pre (&cur)[2][kRuGU], Done done) {
-    if (nb == 1) {
-        // (its own loop: one token's items end with their only block, and
-        // the stream's bookkeeping costs them 3%)
+    if (!MANY || nb == 1) {   // (also a last item's only block)
         float ga[kRuGU], ua[kRuGU];
 #pragma unroll
         for (int r = 0; r < kRuGU; ++r) ga[r] = ua[r] = 0.0f;
@@ -596,7 +594,7 @@ __device__ __forceinline__ void gate_up_rows(const WView& v, int64_t gbase, int 
     }
 }
 
-template <int F, int LPR, bool SH, bool RT>
+template <int F, int LPR, bool SH, bool RT, bool MANY>
 __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_t* lds) {
     constexpr int GPW = kWave / LPR;
     constexpr int RU = kRuGU;
@@ -604,11 +602,12 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
     const int H = a.H, I = a.I, K = a.K;
     const int KS = K + (SH ? 1 : 0);
     const int C = H / Chunk<F>::CH;
-    const int groups = (a.gu_rb + a.gu_nb - 1) / a.gu_nb;   // of gu_nb row blocks
+    const int per = MANY ? a.gu_nb : 1;                     // row blocks per item
+    const int groups = (a.gu_rb + per - 1) / per;
     const int t = j / (KS * groups);
     const int slot = (j / groups) % KS;
-    const int rb = j % groups * a.gu_nb;                    // first row block
-    const int nb = min(a.gu_nb, a.gu_rb - rb);
+    const int rb = j % groups * per;                        // first row block
+    const int nb = min(per, a.gu_rb - rb);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int sub = lane % LPR;
@@ -666,7 +665,7 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
     // (4) the activations into LDS while the weights are in flight
     const bool lo_pass = x_store<F>(xr, H, lds);
     GRIM_TS(a, 1, 2);
-    __shared__ float hrow[kGuMaxNB * kGemvWaves * kWave / 8 * RU];   // this item's rows (fmt_h)
+    __shared__ float hrow[(MANY ? kGuMaxNB : 1) * kGemvWaves * kWave / 8 * RU];   // this item's rows (fmt_h)
     auto done = [&](int blk, const float (&ga)[RU], const float (&ua)[RU]) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < RU; ++r) {
@@ -682,8 +681,8 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
         }
     };
     if (active) {
-        if (lo_pass) gate_up_rows<F, LPR, true>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
-        else gate_up_rows<F, LPR, false>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
+        if (lo_pass) gate_up_rows<F, LPR, true, MANY>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
+        else gate_up_rows<F, LPR, false, MANY>(v, gbase, i0, RB, nb, I, C, sub, lds, H, cur, done);
     } else {
         const float zero[RU] = {};
         for (int blk = 0; blk < nb; ++blk) done(blk, zero, zero);
@@ -717,7 +716,8 @@ __device__ __forceinline__ void gate_up_item(const DecodeArgs& a, int j, uint32_
 // for each of its kPairsDN (slot, row) pairs, all requested at once.
 constexpr int kDnBatch = 3;
 
-template <int F, int LPR>
+// wbase: the slot's first weight row (MANY), or the one row itself.
+template <int F, int LPR, bool MANY>
 __device__ __forceinline__ void down_issue(const DecodeArgs& a, const bool* pvalid,
                                            const bool* pshared, const int64_t* wbase, const int* prow, int o0,
                                            int C, int c0, Pre (&w)[kDnBatch][kPairsDN]) {
@@ -730,24 +730,25 @@ __device__ __forceinline__ void down_issue(const DecodeArgs& a, const bool* pval
         const int cc = c < C ? c : C - 1;
 #pragma unroll
         for (int q = 0; q < kPairsDN; ++q)
-            prefetch<F>(pshared[q] ? a.sdn : a.dn, pvalid[q] ? wbase[q] + min(o0 + prow[q], a.H - 1) : 0, cc, w[b][q]);
+            prefetch<F>(pshared[q] ? a.sdn : a.dn, pvalid[q] ? wbase[q] + (MANY ? min(o0 + prow[q], a.H - 1) : 0) : 0,
+                        cc, w[b][q]);
     }
 }
 
 // nb row blocks of rstep rows from row o0, their chunk batches one stream
 // with the next batch in flight; w holds the first.  done takes each
-// block's sums.
-template <int F, int LPR, bool LO, class Done>
+// block's sums.  !MANY: nb is 1.
+template <int F, int LPR, bool LO, bool MANY, class Done>
 __device__ __forceinline__ void down_rows(const DecodeArgs& a, const int* pslot, const bool* pvalid,
                                           const bool* pshared, const int64_t* wbase, const int* prow, int o0,
                                           int rstep, int nb, int C, int sub, const uint32_t* act, int n,
                                           Pre (&w)[kDnBatch][kPairsDN], Done done) {
-    if (nb == 1) {   // (as in gate_up_rows)
+    if (!MANY || nb == 1) {   // (as in gate_up_rows)
         float acc[kPairsDN];
 #pragma unroll
         for (int q = 0; q < kPairsDN; ++q) acc[q] = 0.0f;
         for (int c0 = sub; c0 < C; c0 += kDnBatch * LPR) {
-            if (c0 != sub) down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o0, C, c0, w);
+            if (c0 != sub) down_issue<F, LPR, MANY>(a, pvalid, pshared, wbase, prow, o0, C, c0, w);
 #pragma unroll
             for (int b = 0; b < kDnBatch; ++b) {
                 const int c = c0 + b * LPR;
@@ -773,7 +774,7 @@ __device__ __forceinline__ void down_rows(const DecodeArgs& a, const int* pslot,
         Pre nxt[kDnBatch][kPairsDN];
         const bool last = ci + 1 == nc;                   // of this block (uniform)
         if (it > 1)
-            down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o0 + (last ? blk + 1 : blk) * rstep, C,
+            down_issue<F, LPR, MANY>(a, pvalid, pshared, wbase, prow, o0 + (last ? blk + 1 : blk) * rstep, C,
                                sub + (last ? 0 : (ci + 1) * kDnBatch * LPR), nxt);
 #pragma unroll
         for (int b = 0; b < kDnBatch; ++b) {
@@ -807,7 +808,7 @@ __device__ __forceinline__ void down_rows(const DecodeArgs& a, const int* pslot,
 
 // down rows of one (token, row block); (slot, row) pairs per lane group,
 // combined in slot order.
-template <int F, int LPR, bool SH>
+template <int F, int LPR, bool SH, bool MANY>
 __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* lds) {
     constexpr int G = kGemvThreads / LPR;
     constexpr int NP = kPairsDN;
@@ -815,10 +816,11 @@ __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* 
     const int KS = K + (SH ? 1 : 0);
     const int C = I / Chunk<F>::CH;
     const int RB = a.dn_rb;
-    const int blocks = (H + RB - 1) / RB, groups = (blocks + a.dn_nb - 1) / a.dn_nb;   // of dn_nb row blocks
+    const int per = MANY ? a.dn_nb : 1;   // row blocks per item
+    const int blocks = (H + RB - 1) / RB, groups = (blocks + per - 1) / per;
     const int t = j / groups;
-    const int o_base = j % groups * a.dn_nb * RB;
-    const int nb = min(a.dn_nb, blocks - j % groups * a.dn_nb);
+    const int o_base = j % groups * per * RB;
+    const int nb = min(per, blocks - j % groups * per);
     const int grp = threadIdx.x / LPR;
     const int sub = threadIdx.x % LPR;
     const int npairs = KS * RB;
@@ -860,10 +862,14 @@ __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* 
             if (e < 0) pvalid[q] = false;
             else wbase[q] = int64_t(e) * H;
         }
+        if (!MANY) {
+            if (o_base + prow[q] >= H) pvalid[q] = false;
+            wbase[q] += min(o_base + prow[q], H - 1);
+        }
     }
     Pre w[kDnBatch][NP];
     // (2) the first batch of weights, then h into LDS while they fly
-    down_issue<F, LPR>(a, pvalid, pshared, wbase, prow, o_base, C, sub, w);
+    down_issue<F, LPR, MANY>(a, pvalid, pshared, wbase, prow, o_base, C, sub, w);
     float gate_sh = 1.0f;
     if (SH && a.gate_in) gate_sh = a.gate_in[t];
     const bool lo_pass = a.fmt_h ? h_store<F>(hr, hsrc, n, lds)
@@ -877,14 +883,14 @@ __device__ __forceinline__ void down_item(const DecodeArgs& a, int j, uint32_t* 
             if (sub == 0 && p < npairs) part[(blk * KS + pslot[q]) * RB + prow[q]] = pvalid[q] ? v : 0.0f;
         }
     };
-    if (lo_pass) down_rows<F, LPR, true>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
-    else down_rows<F, LPR, false>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
+    if (lo_pass) down_rows<F, LPR, true, MANY>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
+    else down_rows<F, LPR, false, MANY>(a, pslot, pvalid, pshared, wbase, prow, o_base, RB, nb, C, sub, lds, n, w, done);
     GRIM_TS(a, 2, 3);
     __syncthreads();
     for (int r = threadIdx.x; r < nb * RB; r += blockDim.x) {
         const int o = o_base + r;
         if (o >= H) continue;
-        const float* pr = part + (r / RB * KS) * RB + r % RB;
+        const float* pr = part + (MANY ? (r / RB * KS) * RB + r % RB : r);
         float total = 0.0f;
         for (int s = 0; s < K; ++s) {
             const float rw = slot_w[s];
@@ -946,15 +952,20 @@ __global__ __launch_bounds__(kGemvThreads) void moe_router_kernel(DecodeArgs a) 
 // The expert kernels.  gate_up: RT = the items run the top-k from the
 // logits, else they read routes; down reads routes (and h) of earlier
 // launches.
-template <int F, int LPG, bool SH, bool RT>
+// MANY: items of several row blocks, in kernels of their own: their stream
+// takes the INT8 gate_up from five waves per SIMD to four and the down from
+// five to three, which items of one block don't repay (12 tokens x top-4, H
+// 1216, I 768: 44.6 us a layer, 50.2 where one kernel did both).
+template <int F, int LPG, bool SH, bool RT, bool MANY>
 __global__ __launch_bounds__(kGemvThreads) void moe_gate_up_kernel(DecodeArgs a) {
     extern __shared__ uint32_t lds[];
-    gate_up_item<F, LPG, SH, RT>(a, blockIdx.x, lds);
+    gate_up_item<F, LPG, SH, RT, MANY>(a, blockIdx.x, lds);
 }
-template <int F, int LPD, bool SH>
-__global__ __launch_bounds__(kGemvThreads) void moe_down_kernel(DecodeArgs a) {
+// (INT8 down of one block: held to the registers of five waves per SIMD)
+template <int F, int LPD, bool SH, bool MANY>
+__global__ __launch_bounds__(kGemvThreads, F == GRIM_FMT_INT8 && !MANY ? 5 : 1) void moe_down_kernel(DecodeArgs a) {
     extern __shared__ uint32_t lds[];
-    down_item<F, LPD, SH>(a, blockIdx.x, lds);
+    down_item<F, LPD, SH, MANY>(a, blockIdx.x, lds);
 }
 
 // ------------------------------------------------------------ launching
@@ -985,13 +996,13 @@ inline hipError_t launch_t(hipStream_t st, const DecodeArgs& a) {
             wave_done = true;
         }
     }
-    if (wave_done) {
-    } else if (a.NG && a.route_topk)
-        hipLaunchKernelGGL((moe_gate_up_kernel<F, LPG, SH, true>), dim3(a.NG), dim3(kGemvThreads),
-                           decode_lds_bytes(F, gu), st, a);
-    else if (a.NG)
-        hipLaunchKernelGGL((moe_gate_up_kernel<F, LPG, SH, false>), dim3(a.NG), dim3(kGemvThreads),
-                           decode_lds_bytes(F, gu), st, a);
+    if (a.NG && !wave_done) {
+        const bool many = a.gu_nb > 1;
+        void (*kern)(DecodeArgs) =
+            a.route_topk ? (many ? moe_gate_up_kernel<F, LPG, SH, true, true> : moe_gate_up_kernel<F, LPG, SH, true, false>)
+                         : (many ? moe_gate_up_kernel<F, LPG, SH, false, true> : moe_gate_up_kernel<F, LPG, SH, false, false>);
+        hipLaunchKernelGGL(kern, dim3(a.NG), dim3(kGemvThreads), decode_lds_bytes(F, gu), st, a);
+    }
     bool dn_done = false;
     if constexpr (kWaveGateUp<F>) {
         if (a.ND && a.dn_wave) {
@@ -1007,9 +1018,10 @@ inline hipError_t launch_t(hipStream_t st, const DecodeArgs& a) {
             dn_done = true;
         }
     }
-    if (a.ND && !dn_done)
-        hipLaunchKernelGGL((moe_down_kernel<F, LPD, SH>), dim3(a.ND), dim3(kGemvThreads),
-                           decode_lds_bytes(F, dn), st, a);
+    if (a.ND && !dn_done) {
+        void (*kern)(DecodeArgs) = a.dn_nb > 1 ? moe_down_kernel<F, LPD, SH, true> : moe_down_kernel<F, LPD, SH, false>;
+        hipLaunchKernelGGL(kern, dim3(a.ND), dim3(kGemvThreads), decode_lds_bytes(F, dn), st, a);
+    }
     return hipGetLastError();
 }
 

@@ -37,3 +37,29 @@ def test_slot_blocks(gpu, fmt, tol, T, H, I, E, K, shared):
         gate = torch.sigmoid(wl.x.double() @ gw.double()).float().contiguous()
     want = O.moe_forward(wl.layer.struct(), oe, ow, gate, wl.x)
     assert rel_l2(y.cpu(), want) <= tol
+
+
+@pytest.mark.parametrize("fmt", ["int8", "bf16"])
+@pytest.mark.parametrize("T,H,I,E,K,shared", [(3, 1008, 512, 16, 10, True), (8, 960, 1040, 12, 6, False),
+                                              (6, 912, 272, 8, 8, True)])
+def test_grouped_blocks_same_bits(gpu, fmt, T, H, I, E, K, shared):
+    """Several row blocks an item (all tokens in a call) and one (each token
+    in a call of its own, too few blocks to group): the same bits."""
+    print(f"slot bits {fmt} T={T} H={H} I={I} E={E} K={K} shared={shared}", flush=True)
+    cfg = configs.Config("t", T, H, E, K, I, fmt, shared=shared, shared_gate=shared)
+    wl = configs.make_workload(cfg, "cpu", seed=T + H)
+    Lg, x = wl.layer.to(gpu), wl.x.to(gpu)
+    y, y1 = torch.empty(T, H, device=gpu), torch.empty(T, H, device=gpu)
+    oe = torch.empty(T, K, dtype=torch.int32, device=gpu)
+    ow = torch.empty(T, K, device=gpu)
+    ops.MoeForward(Lg, T, configs.route_params(cfg, None), 1)(x, y, oe, ow)
+    h, gate = torch.empty(1, K + shared, I, device=gpu), torch.empty(1, device=gpu)
+    for t in range(T):
+        s = slice(t, t + 1)
+        if shared:
+            ops.launch_moe_shared_rows(Lg, Lg.shared_gate_w, oe[s], ow[s], x[s], h, gate, y1[s], 1)
+        else:
+            ops.launch_moe_gate_up_batched(Lg, oe[s], x[s], h, 1)
+            ops.launch_moe_down_batched(Lg, oe[s], ow[s], h, y1[s], 1)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y1)
