@@ -99,6 +99,13 @@ int check_layer(const grim_moe_layer* L) {
     return check_weight(&L->down, "down", int64_t(c.num_experts) * c.hidden, c.inter);
 }
 
+// The shared expert's weight `w` beside the routed experts' `routed`.
+int check_shared(const grim_quant_weight* w, const char* name, int64_t rows, int K, const grim_quant_weight& routed) {
+    if (int r = check_weight(w, name, rows, K)) return r;
+    if (w->fmt != routed.fmt) return fail(GRIM_ERR_FORMAT, "shared expert format must match routed experts");
+    return GRIM_OK;
+}
+
 // LDS ceiling of one work-group on gfx950 (160 KiB).
 constexpr size_t kMaxLds = 160 * 1024;
 
@@ -111,10 +118,8 @@ int gemv_common(void* stream, const grim_moe_layer* L, const grim_quant_weight* 
     if (!rex || !x || !h) return fail(GRIM_ERR_ARG, "null routing/x/h");
     const auto& c = L->cfg;
     if (wsh) {
-        r = check_weight(wsh, "shared gate_up", 2 * int64_t(c.inter), c.hidden);
+        r = check_shared(wsh, "shared gate_up", 2 * int64_t(c.inter), c.hidden, L->gate_up);
         if (r) return r;
-        if (wsh->fmt != L->gate_up.fmt)
-            return fail(GRIM_ERR_FORMAT, "shared expert format must match routed experts");
     }
     if (gate_w && !gate_out) return fail(GRIM_ERR_ARG, "gate_w without gate_out");
     DecodeArgs a{};
@@ -147,10 +152,8 @@ int down_common(void* stream, const grim_moe_layer* L, const grim_quant_weight* 
     if (!rex || !rwt || !h || !y) return fail(GRIM_ERR_ARG, "null routing/h/y");
     const auto& c = L->cfg;
     if (wd) {
-        r = check_weight(wd, "shared down", c.hidden, c.inter);
+        r = check_shared(wd, "shared down", c.hidden, c.inter, L->down);
         if (r) return r;
-        if (wd->fmt != L->down.fmt)
-            return fail(GRIM_ERR_FORMAT, "shared expert format must match routed experts");
     }
     DecodeArgs a{};
     a.gu = a.sgu = view(L->gate_up);
@@ -204,6 +207,16 @@ extern "C" {
 
 __attribute__((visibility("hidden"))) void grimoire_moe_set_error_(const char* msg) {
     std::snprintf(g_err, sizeof g_err, "%s", msg);
+}
+
+// What the slot kernels' entry points check of a layer (for forward.cpp,
+// before its first launch).
+__attribute__((visibility("hidden"))) int grimoire_moe_check_slot_layer_(const grim_moe_layer* L) {
+    int r = check_layer(L);
+    if (!r && L->has_shared)
+        r = check_shared(&L->shared_gate_up, "shared gate_up", 2 * int64_t(L->cfg.inter), L->cfg.hidden, L->gate_up);
+    if (!r && L->has_shared) r = check_shared(&L->shared_down, "shared down", L->cfg.hidden, L->cfg.inter, L->down);
+    return r;
 }
 
 const char* grimoire_moe_last_error(void) { return g_err; }

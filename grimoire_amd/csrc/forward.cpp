@@ -169,6 +169,19 @@ bool wreg_ok(const grim_moe_layer* L, int T) {
            L->cfg.num_experts <= kTileListMaxE && int64_t(T) * wreg_x_planes(f) * wreg_kpad(f, H) * 2 < 0x7FFFFFFF;
 }
 
+// The layer's weights hold what the products read: their buffer descriptors
+// are sized from the configuration, `experts` of them (a shard's count).
+// Any other layer goes to the kernels whose entry points check it.
+bool wreg_weights_whole(const grim_moe_layer* L, int64_t experts) {
+    const int64_t H = L->cfg.hidden, I = L->cfg.inter;
+    auto whole = [](const grim_quant_weight& w, int64_t rows, int64_t K) {
+        return w.K == K && w.N >= rows && w.payload && reinterpret_cast<uintptr_t>(w.payload) % 16 == 0 &&
+               (w.scales || w.fmt == GRIM_FMT_BF16);
+    };
+    return whole(L->gate_up, experts * 2 * I, H) && whole(L->down, experts * H, I) &&
+           (!L->has_shared || (whole(L->shared_gate_up, 2 * I, H) && whole(L->shared_down, H, I)));
+}
+
 // ... and the call takes them: MXFP4 and bf16 experts wherever the grouped
 // GEMM would run (1000 tokens of 128 MXFP4 experts, H = I = 2880: 1300 ->
 // 593 us a layer; 150 tokens of 64 bf16 experts: 299 -> 188 us).  INT4
@@ -181,10 +194,10 @@ bool wreg_ok(const grim_moe_layer* L, int T) {
 // Up to 8 tokens the slot kernels are the faster three-launch decode: 8 x
 // top-4, H 4096, I 2048 (410 MB) 117 -> 95 us; 4 x top-4 of them (205 MB)
 // 65 / 64; 8 x top-8, H 2048, I 768 (151 MB) 56 / 57.
-bool use_wreg(const grim_moe_layer* L, int T, int regime) {
+bool use_wreg(const grim_moe_layer* L, int T, int regime, int shard_count) {
     const int64_t R = int64_t(T) * L->cfg.top_k;
     const int f = L->gate_up.fmt;
-    if (!wreg_ok(L, T)) return false;
+    if (!wreg_ok(L, T) || !wreg_weights_whole(L, shard_count > 0 ? shard_count : L->cfg.num_experts)) return false;
     if (f == GRIM_FMT_INT4 || f == GRIM_FMT_INT4_F16) {
         const int64_t expert = 2 * L->cfg.inter * L->gate_up.row_bytes + L->cfg.hidden * L->down.row_bytes;
         const int64_t slot_bytes = (R + (L->has_shared ? T : 0)) * expert;
@@ -321,6 +334,7 @@ extern "C" int grimoire_moe_route_grouped(void*, const float*, const int32_t*, u
                                           int32_t*, int, int, int, int, int, int, int32_t*, void*,
                                           size_t);
 extern "C" const char* grimoire_moe_last_error(void);
+extern "C" int grimoire_moe_check_slot_layer_(const grim_moe_layer* L);
 
 static int ferr(int code, const char* msg);
 
@@ -615,10 +629,10 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
 // grouped kernels.  The others' buffers have to fit as well (the token rows
 // gathered in place make these the smaller ones for MXFP4 and bf16): whether
 // a workspace is large enough does not depend on the products that run.
-static PlanKind plan_kind(const grim_moe_layer* L, int tokens, int regime, size_t bytes) {
+static PlanKind plan_kind(const grim_moe_layer* L, int tokens, int regime, size_t bytes, int shard_count = 0) {
     Plan p{};
     const PlanKind other = use_gemv(L, tokens, regime) ? PlanKind::kSlots : PlanKind::kGrouped;
-    return use_wreg(L, tokens, regime) && carve(L, tokens, other, nullptr, p) <= bytes &&
+    return use_wreg(L, tokens, regime, shard_count) && carve(L, tokens, other, nullptr, p) <= bytes &&
                    carve(L, tokens, PlanKind::kWreg, nullptr, p) <= bytes
                ? PlanKind::kWreg
                : other;
@@ -778,7 +792,7 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
     const auto& c = L->cfg;
     if (L->has_shared && c.shared_inter != c.inter)
         return ferr(GRIM_ERR_SHAPE, "shared_inter must equal inter");
-    const PlanKind kind = plan_kind(L, tokens, regime, workspace_bytes);
+    const PlanKind kind = plan_kind(L, tokens, regime, workspace_bytes, shard_count);
     const bool gemv = kind == PlanKind::kSlots;
     Plan p{};
     const size_t need = carve(L, tokens, kind, nullptr, p);
@@ -808,7 +822,15 @@ static int forward_impl(void* stream, const grim_moe_layer* L, const grim_route_
     const float scaling = (rp && mode != GRIM_ROUTE_SOFTMAX) ? rp->scaling : 1.0f;
     const bool sh = L->has_shared;
 
-    if (gemv && regime != 3 && tokens <= kDecodeMaxTokens && !shard) {
+    const bool decode = gemv && regime != 3 && tokens <= kDecodeMaxTokens && !shard;
+    if (gemv && !decode) {
+        // what the slot kernels' entry points check (of a shard, its own
+        // experts), before anything is launched
+        grim_moe_layer own = *L;
+        if (shard) own.cfg.num_experts = shard_count;
+        if (int bad = grimoire_moe_check_slot_layer_(&own)) return bad;
+    }
+    if (decode) {
         // three launches: router GEMV, gate_up (each item runs its token's
         // top-k; h written in the staged layout), down
         if (sh && (L->shared_gate_up.fmt != L->gate_up.fmt || L->shared_down.fmt != L->down.fmt))
