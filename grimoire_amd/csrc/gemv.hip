@@ -50,7 +50,26 @@ static int down_rows_per_block(int lpr, int KS) {
     return rb > 0 ? rb : 1;
 }
 
+// LDS of a staged vector of n elements: n words (bf16 pairs hi + lo, or fp32)
+// plus one fp32 sum per chunk.
+static size_t act_bytes(int fmt, size_t n) { return (n + n / chunk_elems(fmt)) * sizeof(uint32_t); }
+
+// A CU's LDS, and what the kernels declare beside the dynamic part (gate_up
+// with the top-k, items of one block and of several; down).
+constexpr size_t kCuLds = 160 * 1024, kGuLdsOne = 3072, kGuLdsMany = 4864, kDnLds = 512;
+// Whether grouping leaves a CU as many work-groups as one block an item does,
+// up to two, and one in any case: `one` and `many` are the LDS of a work-group.
+static bool lds_keeps(size_t one, size_t many) {
+    return kCuLds / many >= std::max<size_t>(1, std::min<size_t>(kCuLds / one, 2));
+}
+
 static int gu_rows_per_block(int lpr) { return kGemvWaves * (kWave / lpr) * kRuGU; }
+
+// Dynamic LDS of the down kernel: h of every slot and nb blocks' dots.
+static size_t down_lds(int fmt, const DecodeArgs& a, int nb) {
+    const int KS = a.K + (a.shared ? 1 : 0);
+    return act_bytes(fmt, size_t(KS) * a.I) + size_t(nb) * KS * a.dn_rb * sizeof(float);
+}
 
 void decode_plan(int fmt, DecodeArgs& a, int roles) {
     const int CH = chunk_elems(fmt);
@@ -89,11 +108,16 @@ void decode_plan(int fmt, DecodeArgs& a, int roles) {
     // items still fill the CUs.  Measured, one block an item / grouped: 3
     // tokens x top-10 of 512 INT8 experts, H 2048, I 512, 42.0 / 34.2 us a
     // layer; 12 tokens x top-4 of 64 bf16 ones, I 1024, 121 / 95.
-    auto grouped = [](int64_t units, int blocks, int64_t items, int most) {
+    // (lds: of a work-group of nb blocks; a layer that fits with one block an
+    // item is never refused for the LDS of several)
+    auto grouped = [](int64_t units, int blocks, int64_t items, int most, auto lds) {
         int nb = 1;
-        while (nb < most && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= items) nb *= 2;
+        while (nb < most && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= items && lds_keeps(lds(1), lds(2 * nb)))
+            nb *= 2;
         return nb;
     };
+    auto gu_lds = [&](int nb) { return act_bytes(fmt, a.H) + (nb > 1 ? kGuLdsMany : kGuLdsOne); };
+    auto dn_lds = [&](int nb) { return down_lds(fmt, a, nb) + kDnLds; };
     a.gu_nb = a.dn_nb = 1;
     const int dn_blocks = (a.H + a.dn_rb - 1) / a.dn_rb;
     // gate_up: where the items hold the top-k (with few slots the start is
@@ -105,15 +129,16 @@ void decode_plan(int fmt, DecodeArgs& a, int roles) {
     // 189).
     if (!a.xf) {
         const int64_t units = int64_t(a.M) * KS;
-        if (a.route_topk) a.gu_nb = grouped(units, a.gu_rb, KS <= 3 ? 3 * kSlotItems / 2 : kSlotItems, kGuMaxNB);
-        else if (units * a.gu_rb >= 32 * kSlotItems) a.gu_nb = grouped(units, a.gu_rb, 4 * kSlotItems, kGuMaxNB);
+        if (a.route_topk) a.gu_nb = grouped(units, a.gu_rb, KS <= 3 ? 3 * kSlotItems / 2 : kSlotItems, kGuMaxNB, gu_lds);
+        else if (units * a.gu_rb >= 32 * kSlotItems) a.gu_nb = grouped(units, a.gu_rb, 4 * kSlotItems, kGuMaxNB, gu_lds);
     }
     // down: staging h is most of a start, so blocks of many rows (few slots)
     // gain the least: INT8 (whose one-block kernel has five waves per SIMD)
     // not at all at 16 rows (55 tokens x top-1, H 2752, I 1728: 169 / 175) and
     // from twice the items at 8 (12 x top-4, H 1216, I 768, 912 items: 46 / 48)
     if (!a.dn_wave && !(fmt == GRIM_FMT_INT8 && a.dn_rb >= 16))
-        a.dn_nb = grouped(a.M, dn_blocks, fmt == GRIM_FMT_INT8 && a.dn_rb >= 8 ? 2 * kSlotItems : kSlotItems, kDnMaxNB);
+        a.dn_nb = grouped(a.M, dn_blocks, fmt == GRIM_FMT_INT8 && a.dn_rb >= 8 ? 2 * kSlotItems : kSlotItems, kDnMaxNB,
+                          dn_lds);
     a.NR = (roles & kRoleRouter) ? a.E : 0;
     a.NG = (roles & kRoleGateUp) ? a.M * KS * ((a.gu_rb + a.gu_nb - 1) / a.gu_nb) : 0;
     a.ND = (roles & kRoleDown) ? a.M * ((dn_blocks + a.dn_nb - 1) / a.dn_nb) : 0;
@@ -160,15 +185,10 @@ bool decode_plan_fused(int fmt, DecodeArgs& a) {
 }
 
 size_t decode_lds_bytes(int fmt, const DecodeArgs& a) {
-    const int CH = chunk_elems(fmt);
-    const int KS = a.K + (a.shared ? 1 : 0);
-    // a staged vector of n elements: n words (bf16 pairs hi + lo, or fp32)
-    // plus one fp32 sum per chunk
-    auto act = [&](size_t n) { return (n + n / CH) * sizeof(uint32_t); };
     size_t b = 0;
     if (a.NR) b = std::max(b, size_t(kGemvWaves) * (512 + 64) * sizeof(float));
-    if (a.NG && !a.xf) b = std::max(b, act(size_t(a.H)));
-    if (a.ND && !a.dn_wave) b = std::max(b, act(size_t(KS) * a.I) + size_t(a.dn_nb) * KS * a.dn_rb * sizeof(float));
+    if (a.NG && !a.xf) b = std::max(b, act_bytes(fmt, a.H));
+    if (a.ND && !a.dn_wave) b = std::max(b, down_lds(fmt, a, a.dn_nb));
     return b;
 }
 

@@ -63,3 +63,19 @@ def test_grouped_blocks_same_bits(gpu, fmt, T, H, I, E, K, shared):
             ops.launch_moe_down_batched(Lg, oe[s], ow[s], h, y1[s], 1)
     torch.cuda.synchronize()
     assert torch.equal(y, y1)
+
+
+@pytest.mark.parametrize("fmt,K,I", [("bf16", 16, 2256), ("bf16", 8, 4512), ("int8", 16, 2368)])
+def test_fills_lds(gpu, fmt, K, I):
+    """Activations that leave no LDS for the dots of a second row block, with
+    enough tokens to group."""
+    print(f"slot lds {fmt} K={K} I={I}", flush=True)
+    cfg = configs.Config("t", 8, 1024, K, K, I, fmt)
+    wl = configs.make_workload(cfg, "cpu", seed=I)
+    y = torch.full((8, 1024), float("nan"), device=gpu)
+    oe = torch.empty(8, K, dtype=torch.int32, device=gpu)
+    ow = torch.empty(8, K, device=gpu)
+    ops.MoeForward(wl.layer.to(gpu), 8, configs.route_params(cfg, None), 1)(wl.x.to(gpu), y, oe, ow)
+    torch.cuda.synchronize()
+    want = O.moe_forward(wl.layer.struct(), oe.cpu(), ow.cpu(), None, wl.x)
+    assert rel_l2(y.cpu(), want) <= 2e-5
