@@ -193,7 +193,13 @@ bool wreg_weights_whole(const grim_moe_layer* L, int64_t experts) {
 // top-2, I 768 (58 MB) 34.4 / 34.6; 9 x top-2, H 1024, I 512 (15 MB) 21 / 28.
 // Up to 8 tokens the slot kernels are the faster three-launch decode: 8 x
 // top-4, H 4096, I 2048 (410 MB) 117 -> 95 us; 4 x top-4 of them (205 MB)
-// 65 / 64; 8 x top-8, H 2048, I 768 (151 MB) 56 / 57.
+// 65 / 64; 8 x top-8, H 2048, I 768 (151 MB) 56 / 57.  A shard's slot kernels
+// read only its own routes, so above 8 tokens its line lies higher (shards of
+// 1/8, all routes' bytes): 12 x top-2, H 2048, I 768 (58 MB) 27.7 / 32.5; 9 x
+// top-3, I 640 (54 MB) 31.2 / 34.2; 1/2, 16 x top-2, I 768 (78 MB) 40 / 34; 1/4,
+// 10 x top-6, I 512 (97 MB) 50 / 33.7; 16 x top-3, I 768 (116 MB) 41 / 34.  Up
+// to 8 tokens a shard has no three-launch decode: 4 x top-4, H 4096, I 2048
+// (205 MB), 1/8, 75 -> 44.
 bool use_wreg(const grim_moe_layer* L, int T, int regime, int shard_count) {
     const int64_t R = int64_t(T) * L->cfg.top_k;
     const int f = L->gate_up.fmt;
@@ -202,8 +208,8 @@ bool use_wreg(const grim_moe_layer* L, int T, int regime, int shard_count) {
         const int64_t expert = 2 * L->cfg.inter * L->gate_up.row_bytes + L->cfg.hidden * L->down.row_bytes;
         const int64_t slot_bytes = (R + (L->has_shared ? T : 0)) * expert;
         if (regime != 0 || T <= 1) return false;
-        return R > 64 ? R <= 2 * int64_t(L->cfg.num_experts)
-                      : slot_bytes >= (T > kDecodeMaxTokens ? int64_t(48) << 20 : int64_t(192) << 20);
+        const int64_t least = T <= kDecodeMaxTokens ? 192 : shard_count > 0 ? 64 : 48;   // MiB
+        return R > 64 ? R <= 2 * int64_t(L->cfg.num_experts) : slot_bytes >= least << 20;
     }
     if (regime == 2) return true;
     return regime == 0 && !use_gemv(L, T, 0) &&
