@@ -23,6 +23,9 @@
 #include "common.hpp"
 #include "tiered.hpp"
 
+#include <algorithm>
+#include <cstdint>
+
 namespace grim {
 
 constexpr int kTmThreads = 256;
@@ -581,12 +584,35 @@ static int lanes_for(int chunks) {
 
 // Row blocks per work-group of the staged kernels: as many as leave at least
 // two work-groups per CU.
-constexpr int kTmItems = 512, kTmMaxNB = 16;
-static int tm_nb(int64_t units, int blocks) {
+constexpr int kTmCUs = 256, kTmMaxNB = 16;
+static int tm_nb(int64_t units, int blocks, int most = kTmMaxNB) {
     int nb = 1;
-    while (nb < kTmMaxNB && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= kTmItems) nb *= 2;
+    while (2 * nb <= most && units * ((blocks + 2 * nb - 1) / (2 * nb)) >= 2 * kTmCUs) nb *= 2;
     return nb;
 }
+
+// ... and of the staged down where that leaves one, or where a CU holds one
+// or two work-groups (more than 8 slots: eight waves; long h): the count whose rounds of
+// per_cu work-groups over the chip, each a start (ids -> pointers -> weights,
+// the staging: about two blocks' time) and nb blocks long, take the least.
+// Two work-groups per CU there meant a second round: 1 token, H 2048, I 768,
+// 16 slots: 15.3 us (unstaged 12.7), by rounds 11.0; H 3584, I 640, 8 slots,
+// 896 work-groups for 768 places: 12.0 (11.4) -> 9.4.  1-8 tokens x 1-16
+// slots of nine layers against the unstaged down: 1.31 times its speed on
+// average and 0.82 at least -> 1.44 and 0.97 (0.2 us).
+constexpr int kTmStart = 2;
+static int tm_nb_rounds(int64_t units, int blocks, int per_cu, int most) {
+    const int64_t slots = int64_t(kTmCUs) * per_cu;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int nb = 1; nb <= most && nb <= blocks; ++nb) {
+        const int64_t groups = units * ((blocks + nb - 1) / nb);
+        const int64_t cost = (groups + slots - 1) / slots * (kTmStart + nb);
+        if (cost < least) { least = cost; best = nb; }
+    }
+    return best;
+}
+
 // The staged kernels' LDS limit, two work-groups per CU (the activations in
 // fp32; larger ones are read from memory by the others).
 constexpr size_t kTmStageMax = 80 * 1024;
@@ -637,9 +663,22 @@ hipError_t tmoe_down(hipStream_t st, const TmoeArgs& a) {
     const int need = (a.K + kTmThreads / kWave - 1) / (kTmThreads / kWave);
     const int kw = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
     {
-        const int blocks = (a.H + per_block - 1) / per_block, nb = tm_nb(a.M, blocks);
-        const size_t lds = size_t(a.K) * (stage_floats(a.I) + nb * per_block) * 4;
-        if (a.K <= 16 && lds <= kTmStageMax) {
+        const int C = a.I / 32, blocks = (a.H + per_block - 1) / per_block;
+        const size_t h_lds = size_t(a.K) * stage_floats(a.I) * 4, block_lds = size_t(a.K) * per_block * 4;
+        const int most = h_lds + block_lds > kTmStageMax ? 0 : int(std::min<size_t>(kTmMaxNB, (kTmStageMax - h_lds) / block_lds));
+        // work-groups per CU: the registers of five of four waves with one
+        // slot each, three with two, one of eight waves; or the staged h
+        const int per_cu = std::min(a.K <= 4 ? 5 : a.K <= 8 ? 3 : 1, std::max(1, int(2 * kTmStageMax / (h_lds + 1024))));
+        int nb = per_cu <= 2 ? 1 : tm_nb(a.M, blocks, most);
+        if (nb == 1) nb = tm_nb_rounds(a.M, blocks, per_cu, most);
+        // one block a work-group, rows that leave three of eight lanes idle
+        // and slots that fill the waves: nothing is saved by the staging (1
+        // token, H 1280, I 1152: 3 / 4 / 7 / 8 slots 5.3 / 5.7 / 8.9 / 8.9 us
+        // unstaged, 5.7 / 6.0 / 9.0 / 9.2 staged; 2 / 5 / 6 slots 5.2 / 8.8 / 8.7,
+        // 4.7 / 8.2 / 8.6)
+        const bool idle = nb == 1 && lpr == 64 && 8 * C <= 5 * lpr && (a.K % 4 == 0 || a.K % 4 == 3);
+        if (a.K <= 16 && most > 0 && !idle) {
+            const size_t lds = h_lds + nb * block_lds;
             const dim3 sgrid(unsigned(int64_t(a.M) * ((blocks + nb - 1) / nb)));
 #define GRIM_TMD_GO(L, KW, NW) \
     hipLaunchKernelGGL((tmoe_down_staged<L, KW, NW>), sgrid, dim3(NW * kWave), lds, st, a, nb)

@@ -3,7 +3,8 @@ where the staged kernels' items can go wrong: enough tokens that a work-group
 takes several row blocks, a last group and a last block partly filled, 1, 2
 and 4 x 4 slots over four and eight waves, rows of several chunk iterations,
 skipped slots; and a down too wide to stage.  Outputs within 1e-5 of the
-largest (fp32 sums in another order)."""
+largest (fp32 sums in another order); a token's bits do not depend on the
+batch, and so not on the kernel or the row blocks per work-group."""
 import numpy as np
 import pytest
 import torch
@@ -37,3 +38,28 @@ def test_tmoe_staged(gpu, H, I, K, E, M):
     for got, want in ((hc, O.tmoe_gate_up(blocks_np, H, I, K, ex, x, M)),
                       (y.cpu().numpy(), O.tmoe_down(blocks_np, H, I, K, ex, w, hc, M))):
         assert np.abs(got - want).max() <= 1e-5 * max(np.abs(want).max(), 1e-30)
+
+
+@pytest.mark.parametrize("H,I,K,E,M", [(1280, 1152, 4, 6, 7), (1280, 1152, 16, 20, 4), (1024, 384, 8, 9, 40),
+                                       (2048, 768, 9, 12, 5), (384, 2176, 2, 4, 600)])
+def test_tmoe_bits_do_not_depend_on_the_batch(gpu, H, I, K, E, M):
+    """One token takes other row blocks per work-group than M do, and at 1280
+    x 1152, 4 slots, the unstaged down."""
+    print(f"tmoe batch bits H={H} I={I} K={K} E={E} M={M}", flush=True)
+    rng = np.random.default_rng(H + I + M)
+    lay = O.tmoe_layout(H, I)
+    layer = tiered.TieredLayer(H, I, K, [torch.from_numpy(make_block(lay, rng)).to(gpu) for _ in range(E)], gpu)
+    ex = torch.from_numpy(np.stack([rng.permutation(E)[:K] for _ in range(M)]).astype(np.int32)).to(gpu)
+    w = torch.from_numpy(rng.random((M, K)).astype(np.float32)).to(gpu)
+    x = torch.from_numpy(rng.standard_normal((M, H)).astype(np.float32)).to(gpu)
+
+    def run(lo, hi):
+        h = torch.full((hi - lo, K * I), float("nan"), device=gpu)
+        y = torch.full((hi - lo, H), float("nan"), device=gpu)
+        layer.gate_up(ex[lo:hi], x[lo:hi], h)
+        layer.down(ex[lo:hi], w[lo:hi], h, y)
+        return h, y
+    h, y = run(0, M)
+    for t in sorted({0, M // 2, M - 1}):
+        h1, y1 = run(t, t + 1)
+        assert torch.equal(h1[0], h[t]) and torch.equal(y1[0], y[t]), t
