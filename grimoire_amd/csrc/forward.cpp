@@ -209,7 +209,9 @@ bool use_wreg(const grim_moe_layer* L, int T, int regime, int shard_count) {
         const int64_t slot_bytes = (R + (L->has_shared ? T : 0)) * expert;
         if (regime != 0 || T <= 1) return false;
         const int64_t least = T <= kDecodeMaxTokens ? 192 : shard_count > 0 ? 64 : 48;   // MiB
-        return R > 64 ? R <= 2 * int64_t(L->cfg.num_experts) : slot_bytes >= least << 20;
+        // (above 64 routes no other path takes rows with a stride, and such a
+        // layer stays refused; the slot kernels, and so this, do below)
+        return R > 64 ? R <= 2 * int64_t(L->cfg.num_experts) && gv_ok(L) : slot_bytes >= least << 20;
     }
     if (regime == 2) return true;
     return regime == 0 && !use_gemv(L, T, 0) &&

@@ -4,6 +4,8 @@ counts around the 16 / 32 / 64 / 128-row blocks, one expert with every token
 and experts with none, K and N with half-filled last segments, scale rows
 whose last window is read early, signed and missing INT4 zero points,
 activations that need their low halves, and a shared expert."""
+import dataclasses
+
 import pytest
 import torch
 
@@ -127,3 +129,31 @@ def test_graph_replays(gpu, fmt, T, regime):
                 g.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, ye), f"replay {rep}"
+
+
+def _widen(w):
+    """The weight with 16 bytes of other rows' codes behind each row."""
+    p = torch.cat((w.payload, w.payload.flip(0)[:, :16]), 1).contiguous()
+    return Weight(w.fmt, w.N, w.K, p, w.scales, w.zeros, w.row_scales)
+
+
+def test_int4_rows_with_a_stride(gpu):
+    """Up to 64 routes such rows give the packed rows' values (16 tokens: the
+    rule on bytes): the same products, but rows of whole kilobytes start their
+    K walk at another place per column tile, so the fp32 sums of 2048 terms
+    run in another order (a bound as for the oracle); above, no path but this one could take them and the call
+    ends in the format error it always had."""
+    cfg = configs.Config("t", 35, 2048, 36, 2, 768, "int4")
+    L = configs.make_layer(cfg, "cpu", seed=3).to(gpu)
+    wide = dataclasses.replace(L, gate_up=_widen(L.gate_up), down=_widen(L.down))
+    x = configs.make_x(cfg, "cpu", seed=3).to(gpu)
+    rp = configs.route_params(cfg, None)
+    y, yw = torch.empty(16, cfg.H, device=gpu), torch.empty(16, cfg.H, device=gpu)
+    ops.MoeForward(L, 16, rp)(x[:16], y)
+    ops.MoeForward(wide, 16, rp)(x[:16], yw)
+    assert rel_l2(yw.cpu(), y.cpu()) <= TOL
+    y = torch.empty(35, cfg.H, device=gpu)
+    ops.MoeForward(L, 35, rp)(x, y)
+    with pytest.raises(_abi.GrimoireError):
+        ops.MoeForward(wide, 35, rp)(x, y)
+    torch.cuda.synchronize()
