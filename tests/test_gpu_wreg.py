@@ -3,7 +3,8 @@ and INT4 batches) against the oracle where their tiles can go wrong: row
 counts around the 16 / 32 / 64 / 128-row blocks, one expert with every token
 and experts with none, K and N with half-filled last segments, scale rows
 whose last window is read early, signed and missing INT4 zero points,
-activations that need their low halves, and a shared expert."""
+activations that need their low halves, both INT4 scale formats, every routing
+mode in the dispatch launch, and a shared expert."""
 import dataclasses
 
 import pytest
@@ -157,3 +158,52 @@ def test_int4_rows_with_a_stride(gpu):
     with pytest.raises(_abi.GrimoireError):
         ops.MoeForward(wide, 35, rp)(x, y)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("H,I", [(512, 640), (2688, 896)])
+@pytest.mark.parametrize("zeros", [None, 0.0, 0.5])
+def test_int4_bf16_scales(gpu, H, I, zeros):
+    """The format that ingestion writes by default: bf16 scales, a zero point
+    per group (some 0xFF: signed codes), or none (zero point 0)."""
+    print(f"wreg int4 bf16 scales H={H} I={I} zeros={zeros}", flush=True)
+    cfg = configs.Config("t", 35, H, 36, 2, I, "int4", shared=True)
+    wl = configs.make_workload(cfg, "cpu", seed=H)
+    L, g = wl.layer, torch.Generator().manual_seed(H)
+    for name in ("gate_up", "down", "shared_gate_up", "shared_down"):
+        w = getattr(L, name)
+        z = None
+        if zeros is not None:
+            z = torch.randint(0, 16, w.scales.shape, dtype=torch.uint8, generator=g)
+            z[torch.rand(z.shape, generator=g) < zeros] = 0xFF
+        sc = w.scales.view(torch.float16).bfloat16().view(torch.int16)
+        setattr(L, name, Weight(_abi.FMT_INT4, w.N, w.K, w.payload, sc, z, w.row_scales))
+    y = torch.full((cfg.T, H), float("nan"), device=gpu)
+    oe = torch.empty(cfg.T, cfg.K, dtype=torch.int32, device=gpu)
+    ow = torch.empty(cfg.T, cfg.K, device=gpu)
+    ops.MoeForward(L.to(gpu), cfg.T, configs.route_params(cfg, None))(wl.x.to(gpu), y, oe, ow)
+    torch.cuda.synchronize()
+    assert rel_l2(y.cpu(), O.moe_forward(L.struct(), oe.cpu(), ow.cpu(), None, wl.x)) <= TOL
+
+
+@pytest.mark.parametrize("route", [_abi.ROUTE_SOFTMAX, _abi.ROUTE_SIGMOID, _abi.ROUTE_GROUP])
+@pytest.mark.parametrize("fmt,T,regime", [("int4", 16, 0), ("int4", 11, 0), ("bf16", 13, 2), ("mxfp4", 1, 2)])
+def test_topk_in_the_dispatch_launch(gpu, fmt, T, regime, route):
+    """Up to 16 tokens the top-k runs in the dispatch launch: its experts and
+    weights are the bits of the slot path's top-k, in each routing mode."""
+    print(f"wreg route fmt={fmt} T={T} route={route}", flush=True)
+    cfg = configs.Config("t", T, 2048, 64, 4, 896, fmt, route=route, bias_std=0.05, scaling=2.5,
+                         n_group=8 if route == _abi.ROUTE_GROUP else 0, topk_group=3 if route == _abi.ROUTE_GROUP else 0)
+    wl = configs.make_workload(cfg, "cpu", seed=T + route)
+    bias = None if wl.route_bias is None else wl.route_bias.to(gpu)
+    L, x = wl.layer.to(gpu), wl.x.to(gpu)
+    got = []
+    for r in (regime, 3):
+        y = torch.full((T, cfg.H), float("nan"), device=gpu)
+        oe = torch.empty(T, cfg.K, dtype=torch.int32, device=gpu)
+        ow = torch.empty(T, cfg.K, device=gpu)
+        ops.MoeForward(L, T, configs.route_params(cfg, bias), r)(x, y, oe, ow)
+        got.append((y, oe, ow))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+    want = O.moe_forward(wl.layer.struct(), got[0][1].cpu(), got[0][2].cpu(), None, wl.x)
+    assert rel_l2(got[0][0].cpu(), want) <= TOL
