@@ -1,7 +1,7 @@
 """The K-split router for 33 tokens up to one round of its tiles: logits
 against the oracle at ragged token / expert / K-part edges (K parts of unequal
 length, waves without any), x that is not bf16 valued in some units, both tile
-widths and just past the last one; and the forward's routing, which adds the
+widths and just past the last one, and the kernels behind it; and the forward's routing, which adds the
 two K halves in the top-k, from the same bits."""
 import pytest
 import torch
@@ -29,6 +29,20 @@ def test_router_k16(gpu, T, E, H, kind):
     ops.router_logits(W.to(gpu), x.to(gpu), out)
     torch.cuda.synchronize()
     # three limbs keep 24 bits of each operand; sums of H products in fp32
+    assert rel_l2(out.cpu(), x.double() @ W.double().T) < 1e-6
+
+
+@pytest.mark.parametrize("T,E,H", [(4200, 64, 128), (40, 4200, 256), (4161, 65, 96), (97, 2070, 100)])
+def test_router_past_one_round(gpu, T, E, H):
+    """More tiles than CUs and no K long enough for the split of long
+    prompts: the 64 x 64 tiles, and H that is no whole number of K tiles."""
+    print(f"router past one round T={T} E={E} H={H}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    W = torch.randn(E, H, generator=g) * 0.02
+    x = torch.randn(T, H, generator=g)
+    out = torch.full((T, E), float("nan"), device=gpu)
+    ops.router_logits(W.to(gpu), x.to(gpu), out)
+    torch.cuda.synchronize()
     assert rel_l2(out.cpu(), x.double() @ W.double().T) < 1e-6
 
 
