@@ -373,7 +373,7 @@ def edges_bench(dev, stream, reps=20):
                      "-> INT4 bf16 scales, device-resident sources",
             "ms": round(ms, 3), "host_ms": round(host_ms, 3), "bytes": src_bytes + dst_bytes,
             "gbs": round((src_bytes + dst_bytes) / (ms * 1e-3) / 1e9, 1),
-            "note": "two batched calls (gate+up, down), 64 GPTQ projections per launch"}
+            "note": "two batched calls (gate+up, down), 128 GPTQ projections per launch"}
         res["tiered_nvfp4"] = _tiered_bench(dev, stream, timed)
     return res
 

@@ -184,7 +184,10 @@ bool wreg_weights_whole(const grim_moe_layer* L, int64_t experts) {
 
 // ... and the call takes them: MXFP4 and bf16 experts wherever the grouped
 // GEMM would run (1000 tokens of 128 MXFP4 experts, H = I = 2880: 1300 ->
-// 593 us a layer; 150 tokens of 64 bf16 experts: 299 -> 188 us).  INT4
+// 606 us a layer; 150 tokens of 64 bf16 experts: 299 -> 188 us; many rows per
+// expert too: 4096 tokens x top-8 of 32 MXFP4 experts, H = I = 2880: 2509 ->
+// 2127, of 16 bf16 ones, H 2048, I 1024: 997 -> 806; sixty layers of 33 to
+// 4096 tokens: 1.18 to 4.5 times the tile kernel's speed).  INT4
 // experts, up to the two routes per expert that INT4 batches are taken for:
 // above 64 routes always (the vector-ALU grouped GEMV otherwise: 20 tokens x
 // top-8 of 128, H 2048, I 768: 304 -> 76 us), below when the bytes that the

@@ -38,8 +38,9 @@ struct WregArgs {
 bool wreg_weight_ok(const grim_quant_weight& w, int rows_per_expert, int K);
 // Reduction length padded to whole segments of the format.
 int wreg_kpad(int fmt, int K);
-// Activation planes of gate_up: INT4 experts split fp32 x exactly in two
-// bf16 halves, the others round x to bf16.
+// Activation planes of gate_up: INT4 experts split fp32 x in two bf16 halves
+// (exact for 16 significant bits, within 2^-17 of x otherwise), the others
+// round x to bf16.
 int wreg_x_planes(int fmt);
 // x fp32 [T][H] -> bf16 rows [T][planes][wreg_kpad] (+ per row lo != 0), and
 // in the same launch the dispatch of the routes in tk.out_e (its first

@@ -364,7 +364,7 @@ int grimoire_moe_ingest_projection(void* stream, const grim_expert_src* src,
                                    const grim_quant_weight* dst, int row0);
 /* n projections of one kind and shape (host arrays src[n], row0[n]) into
  * the same stacked weight, e.g. every expert's gate and up of a layer:
- * GPTQ sources go 64 per launch.  Same conversions and rules as above. */
+ * GPTQ sources go 128 per launch.  Same conversions and rules as above. */
 int grimoire_moe_ingest_projections(void* stream, const grim_expert_src* srcs,
                                     const int32_t* row0, int n, const grim_quant_weight* dst);
 
