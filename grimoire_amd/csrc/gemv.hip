@@ -13,6 +13,8 @@ constexpr int kPairsDN = 2;
 // Items the slot kernels keep at least when they group row blocks (two per
 // CU), and row blocks per down item at most.
 constexpr int kSlotItems = 512, kDnMaxNB = 16;
+// One round of gate_up's single-block work-groups: five a CU.
+constexpr int kOneRound = 5 * 256;
 
 hipError_t decode_launch_fmt_0(hipStream_t, const DecodeArgs&);
 hipError_t decode_launch_fmt_3(hipStream_t, const DecodeArgs&);
@@ -120,16 +122,19 @@ void decode_plan(int fmt, DecodeArgs& a, int roles) {
     auto dn_lds = [&](int nb) { return down_lds(fmt, a, nb) + kDnLds; };
     a.gu_nb = a.dn_nb = 1;
     const int dn_blocks = (a.H + a.dn_rb - 1) / a.dn_rb;
-    // gate_up: where the items hold the top-k (with few slots the start is
-    // short: 4 tokens x top-2, H 3584, I 896 in 672 items 46.7 us, ungrouped
-    // 42.6), or there are a great many (30 tokens x top-2 + shared of 16 bf16
-    // experts, H 2432, I 1536: 17280 items, 340 / 302 us).  Otherwise the
+    // gate_up: where the items hold the top-k and single blocks are more than
+    // one round of the chip (3 tokens x top-4 + shared, H 1152, I 576, 1080
+    // items: INT8 9.3 / 9.9 us, bf16 11.0 / 12.2; 4 tokens, 1440 items: 12.9 /
+    // 11.1, 15.6 / 13.7; 130 layers of 1024 to 3100 items against one block:
+    // 1.08 times the speed on average, 0.96 at least, 0.93 without the line at
+    // one round); or there are a great many (30 tokens x top-2 + shared of 16
+    // bf16 experts, H 2432, I 1536: 17280 items, 340 / 302 us).  Otherwise the
     // stream's registers cost what the starts saved (INT8, 25 tokens x top-2 +
     // shared, H 2432, I 960: 117 / 128; bf16, 43 x top-1, H 2240, I 1728: 175 /
     // 189).
     if (!a.xf) {
         const int64_t units = int64_t(a.M) * KS;
-        if (a.route_topk) a.gu_nb = grouped(units, a.gu_rb, KS <= 3 ? 3 * kSlotItems / 2 : kSlotItems, kGuMaxNB, gu_lds);
+        if (a.route_topk && units * a.gu_rb > kOneRound) a.gu_nb = grouped(units, a.gu_rb, kSlotItems, kGuMaxNB, gu_lds);
         else if (units * a.gu_rb >= 32 * kSlotItems) a.gu_nb = grouped(units, a.gu_rb, 4 * kSlotItems, kGuMaxNB, gu_lds);
     }
     // down: staging h is most of a start, so blocks of many rows (few slots)
